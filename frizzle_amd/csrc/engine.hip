@@ -101,7 +101,7 @@ struct frz_model {
   float *hidden = nullptr, *hidden_b = nullptr, *normed = nullptr, *qkv = nullptr, *attn = nullptr,
         *output = nullptr, *act = nullptr, *logits = nullptr, *partials = nullptr,
         *stats = nullptr;
-  // A split down product's later range sums (kSplitParts x 16 rows x hidden),
+  // A split down product's later range sums (kSplitParts x kSplitRows rows x hidden),
   // added by the norm that reads its output.
   float* split_parts = nullptr;
   uint32_t *topk_scratch = nullptr, *candidates = nullptr, *sampled = nullptr,

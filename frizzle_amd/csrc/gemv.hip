@@ -560,9 +560,12 @@ bool build_schedule(int groups, Schedule<NB>& S) {
   return t > 0;
 }
 
-// ---- steps of at most 16 rows: a pass a wave ------------------------------
-// A step of at most 16 rows (a batch of variants, a prompt's last rows) makes
-// one 16 x 16 tile per 16 output rows. A workgroup takes a tile and its eight
+// ---- steps of up to a few hundred rows: a pass a wave ----------------------
+// A step of few rows (a batch of variants, a chat message, a prompt's last
+// rows) makes one 16 x 16 tile per 16 output rows and 16 tokens. With a wave
+// a tile (gemm_ranges) its 32 ranges are one serial chain, which is all the
+// time there is until the tiles fill the chip: 55 us for gate and up and 51
+// for down at any 17 to 128 tokens. Here a workgroup takes a tile and its eight
 // waves a pass each. A pass is any four of the 32 ranges, chained in the four
 // blocks of one v_mfma_f32_16x16x1_4b_f32 per k; the range sums meet in LDS
 // by range index and are added in range order, so which ranges share a pass
@@ -696,7 +699,10 @@ __device__ __forceinline__ void lds_reads_done() { __builtin_amdgcn_s_waitcnt(0x
 // one matrix (a pair of tiles on the same inputs).
 constexpr int kPlainKind = 0, kGatedKind = 1, kPairKind = 2;
 
-// Grid: x = 16-row tiles (32-row pairs); y = the halves of a split tile
+// Grid: x = 16-row tiles (32-row pairs); z = 16-token tiles (a row tile's
+// token tiles lie a multiple of eight workgroups apart for the model's
+// shapes, so on one XCD, whose L2 keeps the weights they share); y = the
+// halves of a split tile
 // (HALVES = 2: the workgroup of half h takes passes 4 h .. 4 h + 3, which
 // hold ranges 16 h .. 16 h + 15; half 0 writes their prefix to y, half 1
 // each range's sum to parts). Rows past the end are read clamped and not
@@ -730,6 +736,7 @@ __global__ __launch_bounds__(kPassWaves / HALVES * 64, 4 / HALVES) void pass_til
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int groups = w.cols >> 5;
   const int row0 = (int)blockIdx.x * D * (PAIR ? 2 : 1);
+  const int token0 = (int)blockIdx.z * D;
   float4* const slots[3] = {slot0 + wave * kSlotFloat4s, slot1 + (kSlots > 1 ? wave : 0) * kSlotFloat4s,
                             slot2 + (kSlots > 2 ? wave : 0) * kSlotFloat4s};
 
@@ -737,7 +744,7 @@ __global__ __launch_bounds__(kPassWaves / HALVES * 64, 4 / HALVES) void pass_til
   // table's pin words for the layer, read now and used at the end. Rows of
   // the buffers past the step's tokens are read, not stored.
   const int i_out = t & (D * D - 1);
-  const int tk_out = min(i_out / D, max_tokens - 1);
+  const int tk_out = min(token0 + i_out / D, max_tokens - 1);
   // The step's fields the combine uses, loaded now through vector
   // registers: scalar loads return out of order, so a scalar read of the
   // step would be waited for with the arguments', before the first weight
@@ -809,7 +816,7 @@ __global__ __launch_bounds__(kPassWaves / HALVES * 64, 4 / HALVES) void pass_til
   const uint32_t f_moved = (uint32_t)((lane & 7) ^ (lane >> 3));
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int tok = min(8 * h + (lane >> 3), max_tokens - 1);
+    const int tok = min(token0 + 8 * h + (lane >> 3), max_tokens - 1);
     L.x_off[h] = 4u * (uint32_t)tok * (uint32_t)x_stride + 16u * f_moved;
   }
   L.x_read = 128u * (uint32_t)lane + 16u * (uint32_t)(lane & 7);
@@ -896,7 +903,7 @@ __global__ __launch_bounds__(kPassWaves / HALVES * 64, 4 / HALVES) void pass_til
   }
   __syncthreads();
   if (t >= D * D) return;
-  const int tk = i_out / D, n = row0 + i_out % D;
+  const int tk = token0 + i_out / D, n = row0 + i_out % D;
   if (tk >= (int)step_pt.y || n >= w.rows) return;
   float* yr = y + (size_t)tk * y_stride;
   // Range r's sum for the thread's output (token tk, row i_out % D: at
@@ -971,14 +978,14 @@ hipError_t launch_pass_tiles(hipStream_t s, const DevStep* step, QMatrix w, QMat
   const uint64_t x_bytes = 4ull * (uint64_t)x_stride * (uint64_t)max_tokens;
   const uint64_t codes = (uint64_t)code_bytes(F) * (uint64_t)w.rows * (uint64_t)groups;
   // Every range holds a group; offsets stay below the past-the-end one.
-  if (groups < kRanges || groups >= 0x8000 || max_tokens > Mfma<4>::kDim ||
-      x_bytes >= kPastEnd || codes >= kPastEnd) {
+  if (groups < kRanges || groups >= 0x8000 || x_bytes >= kPastEnd || codes >= kPastEnd) {
     return hipErrorInvalidValue;
   }
+  const int token_tiles = (max_tokens + Mfma<4>::kDim - 1) / Mfma<4>::kDim;
   const int halves = parts ? 2 : 1;
   const PassOrder order = pass_order(groups, halves);
   const int rows_a_block = Mfma<4>::kDim * (KIND == kPairKind ? 2 : 1);
-  const dim3 grid((w.rows + rows_a_block - 1) / rows_a_block, halves);
+  const dim3 grid((w.rows + rows_a_block - 1) / rows_a_block, halves, token_tiles);
   const int threads = kPassWaves / halves * 64;
   // Straight-line forms for the lengths of the model's products (K = 1,024,
   // 1,152 and 6,912); a loop for the others.
@@ -1033,10 +1040,16 @@ hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, QMatrix 
   return hipGetLastError();
 }
 
-// A step of at most 16 rows over K of 32 groups or more (a batch of
-// variants, a prompt's last rows) takes a pass a wave.
+// A step over K of 32 groups or more takes a pass a wave up to kSplitRows
+// rows, where the tiles of a wave each (gemm_ranges) catch up: a layer's
+// products took, a wave a tile then a pass a wave, 142 then 56 us at 32
+// rows, 153 then 125 at 128, 230 then 209 at 256, 378 then 389 at 512 (the
+// decoded weights are shared by 32 tokens there, by 16 here). A matrix of
+// thousands of tiles (the vocabulary's) fills the chip a wave a tile from 17
+// rows on.
 bool pass_tiles(const QMatrix& w, int max_tokens) {
-  return max_tokens <= Mfma<4>::kDim && (w.cols >> 5) >= kRanges;
+  const int most = w.rows < 512 * Mfma<4>::kDim ? kSplitRows : Mfma<4>::kDim;
+  return max_tokens <= most && (w.cols >> 5) >= kRanges;
 }
 
 }  // namespace

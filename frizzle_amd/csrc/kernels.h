@@ -10,7 +10,7 @@ namespace frz {
 
 constexpr int kRanges = 32;        // a row's K-ranges (matmul.h:88-97)
 constexpr int kSplitParts = kRanges / 2;  // range sums a split product leaves apart
-constexpr int kSplitRows = 16;            // most rows a split product takes
+constexpr int kSplitRows = 512;           // most rows a split product takes
 constexpr int kChunkKeys = 64;     // attention chunk (attention.wgsl:60)
 constexpr int kTileKeys = 8;       // attention tile at d = 256
 constexpr int kCandidates = 64;    // top-k kept (residency/plan.h:195)
@@ -97,7 +97,7 @@ inline bool has_members(const QMatrix& w) { return w.split[0] != 0; }
 hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
                        const float* x, int x_stride, float* y, int y_stride,
                        int max_tokens, bool last_token);
-// A step of at most 16 rows over a long K may split each output's 32 ranges
+// A step of at most kSplitRows rows over a long K may split each output's 32 ranges
 // over two workgroups: y then holds the in-order prefix of ranges 0..15 and
 // parts + j * parts_stride (y's row layout) range 16 + j's sum, for the
 // consumer to add in order (NormArgs::parts). gemv_splits says whether

@@ -1,0 +1,65 @@
+"""The products of steps of 2 to 512 rows through the C ABI, bit for bit the
+oracle's, at the edges of their token tiles and of the rules that choose a
+kernel for a step's rows."""
+import numpy as np
+import pytest
+
+import _oracle as orc
+import frizzle_amd as fz
+from helpers import assert_same_bits, format_blocks, q4_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(device, fmt, blocks):
+    codes, scales = fz.block_split(fmt, blocks)
+    return device.array(codes), device.array(scales)
+
+
+def _check_rows(got, want_row, tokens):
+    """Every token's row when they are few; else both edges of each 16-token
+    tile and a stride through the rest."""
+    rows = set(range(tokens)) if tokens <= 40 else (
+        {t for t in range(tokens) if t % 16 in (0, 15)} | set(range(0, tokens, 7)) | {tokens - 1})
+    for t in sorted(rows):
+        assert_same_bits(got[t], want_row(t), f"token {t}")
+
+
+@pytest.mark.parametrize("fmt,rows,cols,tokens", [
+    (2, 1536, 1152, 17), (2, 1152, 1024, 31), (2, 1152, 6912, 33), (2, 100, 1152, 64),
+    (2, 1152, 6912, 256), (2, 1152, 6912, 257), (2, 1536, 1152, 255), (2, 8192, 1152, 17),
+    (2, 8191, 1152, 17), (3, 1152, 6912, 49), (8, 1152, 6912, 130), (3, 40, 1152, 300),
+    (2, 1152, 1056, 19)])
+def test_row_products_bit_exact(device, fmt, rows, cols, tokens):
+    rng = np.random.default_rng(rows + cols + tokens)
+    w = format_blocks(rng, fmt, rows, cols)
+    x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    codes, scales = _dev(device, fmt, w)
+    dx, dy = device.array(x), device.empty((tokens, rows), np.float32)
+    fz._lib.check(fz.load().frz_op_gemv_format(device.handle, fmt, codes.ptr, scales.ptr, rows,
+                                               cols, dx.ptr, cols, dy.ptr, rows, tokens, 0))
+    _check_rows(dy.numpy(), lambda t: orc.gemv_format(fmt, w, rows, cols, x[t]), tokens)
+
+
+@pytest.mark.parametrize("rows,tokens", [(6912, 17), (1000, 48), (96, 256), (96, 257), (100, 512)])
+def test_gated_rows_bit_exact(device, rows, tokens):
+    rng = np.random.default_rng(rows + tokens)
+    cols, layers, layer, position = 1152, 2, 1, 30
+    g, u = q4_blocks(rng, rows, cols), q4_blocks(rng, rows, cols)
+    x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    # Pins that start and end inside the step, at the first and last neurons.
+    edits = [fz.Edit(layer, n, fz.EditKind.SET, 0.5 * n + 1, 3, 3 + tokens // 2)
+             for n in (0, 15, 16, rows - 1)]
+    table = fz.edit_table(edits, layers, origin=position)
+    (gc, gs), (uc, us) = _dev(device, 2, g), _dev(device, 2, u)
+    dx, dt = device.array(x), device.array(table)
+    da = device.empty((tokens, rows), np.float32)
+    fz._lib.check(fz.load().frz_op_gated(device.handle, gc.ptr, gs.ptr, uc.ptr, us.ptr, rows,
+                                         cols, dx.ptr, da.ptr, tokens, position, dt.ptr, layer))
+
+    def want(t):
+        row = orc.gated(g, u, rows, cols, x[t])
+        orc.lib().orc_edit_row(table.ctypes.data, layer, position + t, rows, row.ctypes.data)
+        return row
+
+    _check_rows(da.numpy(), want, tokens)
