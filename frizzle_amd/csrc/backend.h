@@ -3,11 +3,16 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/frizzle_hip.h"
 #include "kernels.h"
+
+namespace frz {
+constexpr size_t kTopkScratchWords = 2 * 64 * (1024 + 64);
+}
 
 struct frz_device {
   int ordinal = 0;
@@ -17,6 +22,11 @@ struct frz_device {
   // This device's copy of the static decode-attention workspace (the
   // address hipGetSymbolAddress gave at frz_open, with this device current).
   float* static_workspace = nullptr;
+  // frz_op_topk's scratch for up to kTopkScratchWords words (a vocabulary of
+  // 1,048,576 logits; longer calls allocate their own): an allocation and
+  // its free, which waits for the device, cost more than the selection.
+  uint32_t* topk_scratch = nullptr;
+  std::mutex ops;  // held while an op enqueues launches that share a buffer here
 };
 
 namespace frz {
@@ -25,8 +35,10 @@ namespace frz {
 int fail(int status, const std::string& message);
 // FRZ_OK, or FRZ_ERR_DEVICE with the HIP error's text.
 int check_hip(hipError_t e, const char* what);
-// Copies a step record to the device and waits.
+// Puts a step record without its ids on the device, in stream order.
 int device_put_step(frz_device* dev, const DevStep& s);
+// Copies a whole step record to the device and waits.
+int device_copy_step(frz_device* dev, const DevStep& s);
 // Reports a launch's error, else waits for the stream.
 int device_finish(frz_device* dev, hipError_t launched, const char* what);
 // The sampling settings into a step record (sampler::apply,
