@@ -46,8 +46,7 @@ __device__ __forceinline__ float half_to_float(uint16_t h) {
 // token's inputs for that group. So every lane does distinct work and a pass
 // keeps NB chains in flight. The inputs of a step (NB groups x D tokens = 64
 // lines of 32 floats) are loaded whole-line into LDS and read back one line
-// per lane. A gated wave holds the gate and up tiles of the same neurons,
-// sharing the inputs.
+// per lane.
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
@@ -225,12 +224,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* base, ui
 constexpr int kXLine = 9;
 constexpr int kXBuf = 64 * kXLine;
 
-template <int NB, bool GATED>
+template <int NB>
 struct Tile {
   static constexpr int D = Mfma<NB>::kDim;
   static constexpr int kTokenRows = 8 / NB;  // distinct tokens a lane loads
-  static constexpr int kMats = GATED ? 2 : 1;
-  __amdgpu_buffer_rsrc_t x, codes[kMats], scales[kMats];
+  __amdgpu_buffer_rsrc_t x, codes, scales;
   uint32_t x_off[kTokenRows];  // byte offset of float4 lane % 8 of each token it loads
   uint32_t row_group0;         // this lane's row times the row's groups
   float4* x_put;               // its load slots (+ 8 kXLine i)
@@ -241,10 +239,10 @@ struct Tile {
 // Step t's inputs: instruction i is lines 8 i .. 8 i + 7, block
 // i / (8 / NB). A finished block's lines are loaded (from a valid group)
 // and zeroed when staged.
-template <int NB, bool GATED>
-__device__ __forceinline__ void load_inputs(const Tile<NB, GATED>& T, const StepInfo<NB>& I,
+template <int NB>
+__device__ __forceinline__ void load_inputs(const Tile<NB>& T, const StepInfo<NB>& I,
                                             float4 (&G)[8]) {
-  constexpr int kPer = Tile<NB, GATED>::kTokenRows;
+  constexpr int kPer = Tile<NB>::kTokenRows;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const uint32_t g = I.entry(i / kPer) & 0x7FFFu;
@@ -253,10 +251,10 @@ __device__ __forceinline__ void load_inputs(const Tile<NB, GATED>& T, const Step
   }
 }
 
-template <int NB, bool GATED>
-__device__ __forceinline__ void stage_inputs(const Tile<NB, GATED>& T, const StepInfo<NB>& I,
+template <int NB>
+__device__ __forceinline__ void stage_inputs(const Tile<NB>& T, const StepInfo<NB>& I,
                                              float4 (&G)[8]) {
-  constexpr int kPer = Tile<NB, GATED>::kTokenRows;
+  constexpr int kPer = Tile<NB>::kTokenRows;
   if (I.flags & kPads) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -267,12 +265,12 @@ __device__ __forceinline__ void stage_inputs(const Tile<NB, GATED>& T, const Ste
   for (int i = 0; i < 8; ++i) T.x_put[8 * kXLine * i] = G[i];
 }
 
-// A lane's weights for a step: one group of each matrix. A gated product's
-// matrices are Q4_0; a plain one's may be Q4_1 or Q8_0 as well.
-template <bool GATED, int F>
+// A lane's weights for a step: a group of one matrix, or of each of two (TWO:
+// gate and up, or a pair of tiles), which are Q4_0.
+template <bool TWO, int F>
 struct Weights {
-  uint4 c[GATED ? 2 : 1];
-  uint16_t d[GATED ? 2 : 1];
+  uint4 c[TWO ? 2 : 1];
+  uint16_t d[TWO ? 2 : 1];
 };
 template <>
 struct Weights<false, kQ8_0> {
@@ -285,60 +283,50 @@ struct Weights<false, kQ4_1> {
   uint32_t d[1];  // d, then m in the high half
 };
 
-template <int NB, bool GATED, int F>
-__device__ __forceinline__ void load_weights(const Tile<NB, GATED>& T, const StepInfo<NB>& I,
-                                             Weights<GATED, F>& W) {
+template <int NB, int F>
+__device__ __forceinline__ void load_weights(const Tile<NB>& T, const StepInfo<NB>& I,
+                                             Weights<false, F>& W) {
   // this lane's block's group
   uint32_t g = I.entry(0);
 #pragma unroll
   for (int b = 1; b < NB; ++b) g = T.block == b ? I.entry(b) : g;
   const uint32_t blk = T.row_group0 + (g & 0x7FFFu);
-#pragma unroll
-  for (int m = 0; m < Tile<NB, GATED>::kMats; ++m) {
-    if constexpr (F == kQ8_0) {
-      W.c[0] = __builtin_bit_cast(uint4,
-                                  __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 32 * blk, 0, 0));
-      W.c[1] = __builtin_bit_cast(
-          uint4, __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 32 * blk + 16, 0, 0));
-      W.d[0] = __builtin_amdgcn_raw_buffer_load_b16(T.scales[m], 2 * blk, 0, 0);
-    } else if constexpr (F == kQ4_1) {
-      W.c[0] = __builtin_bit_cast(uint4,
-                                  __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 16 * blk, 0, 0));
-      W.d[0] = __builtin_amdgcn_raw_buffer_load_b32(T.scales[m], 4 * blk, 0, 0);
-    } else {
-      W.c[m] = __builtin_bit_cast(uint4,
-                                  __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 16 * blk, 0, 0));
-      W.d[m] = __builtin_amdgcn_raw_buffer_load_b16(T.scales[m], 2 * blk, 0, 0);
-    }
+  const uint32_t code_at = (uint32_t)code_bytes(F) * blk;
+  W.c[0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(T.codes, code_at, 0, 0));
+  if constexpr (F == kQ8_0) {
+    W.c[1] = __builtin_bit_cast(
+        uint4, __builtin_amdgcn_raw_buffer_load_b128(T.codes, code_at + 16, 0, 0));
+  }
+  if constexpr (F == kQ4_1) {
+    W.d[0] = __builtin_amdgcn_raw_buffer_load_b32(T.scales, 4 * blk, 0, 0);
+  } else {
+    W.d[0] = __builtin_amdgcn_raw_buffer_load_b16(T.scales, 2 * blk, 0, 0);
   }
 }
 
-// Products for k = 16 H .. 16 H + 15 of a step, per matrix: decode the
-// weights, then the 16 products per block.
-template <int NB, bool GATED, int F, int H>
-__device__ __forceinline__ void chain_half(const float4 (&xv)[8], const Weights<GATED, F>& W,
-                                           typename Mfma<NB>::Acc (&acc)[GATED ? 2 : 1]) {
-#pragma unroll
-  for (int m = 0; m < (GATED ? 2 : 1); ++m) {
-    float wk[16];
-    if constexpr (F == kQ8_0) {
-      decode_half_q8_0(W.c[H], W.d[0], wk);
-    } else if constexpr (F == kQ4_1) {
-      decode_half_q4_1<H>(W.c[0], W.d[0], wk);
-    } else {
-      decode_half<H>(W.c[m], W.d[m], wk);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float4 x4 = xv[4 * H + i];
-      acc[m] = Mfma<NB>::op(wk[4 * i + 0], x4.x, acc[m]);
-      acc[m] = Mfma<NB>::op(wk[4 * i + 1], x4.y, acc[m]);
-      acc[m] = Mfma<NB>::op(wk[4 * i + 2], x4.z, acc[m]);
-      acc[m] = Mfma<NB>::op(wk[4 * i + 3], x4.w, acc[m]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
+// Products for k = 16 H .. 16 H + 15 of a step: decode the weights, then the
+// 16 products per block.
+template <int NB, int F, int H>
+__device__ __forceinline__ void chain_half(const float4 (&xv)[8], const Weights<false, F>& W,
+                                           typename Mfma<NB>::Acc& acc) {
+  float wk[16];
+  if constexpr (F == kQ8_0) {
+    decode_half_q8_0(W.c[H], W.d[0], wk);
+  } else if constexpr (F == kQ4_1) {
+    decode_half_q4_1<H>(W.c[0], W.d[0], wk);
+  } else {
+    decode_half<H>(W.c[0], W.d[0], wk);
   }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float4 x4 = xv[4 * H + i];
+    acc = Mfma<NB>::op(wk[4 * i + 0], x4.x, acc);
+    acc = Mfma<NB>::op(wk[4 * i + 1], x4.y, acc);
+    acc = Mfma<NB>::op(wk[4 * i + 2], x4.z, acc);
+    acc = Mfma<NB>::op(wk[4 * i + 3], x4.w, acc);
+  }
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // Two Q4_0 chains on the same inputs (gate and up, or two tiles), quarter Q
@@ -378,11 +366,11 @@ __device__ __forceinline__ void chain_half_two(const float4 (&xv)[8], const Weig
 // chain this step's 32 products per block, half a group at a time so that
 // the decoded weights need few registers. Vector instructions do not run
 // beside the fp32 matrix instructions, so each kind is kept in runs.
-template <int NB, bool GATED, int F>
-__device__ __forceinline__ void chain_step(const Tile<NB, GATED>& T, const StepInfo<NB>& I1,
+template <int NB, int F>
+__device__ __forceinline__ void chain_step(const Tile<NB>& T, const StepInfo<NB>& I1,
                                            const StepInfo<NB>& I2, float4 (&G)[8],
-                                           const Weights<GATED, F>& W, Weights<GATED, F>& W_next,
-                                           typename Mfma<NB>::Acc (&acc)[GATED ? 2 : 1]) {
+                                           const Weights<false, F>& W, Weights<false, F>& W_next,
+                                           typename Mfma<NB>::Acc& acc) {
   float4 xv[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) xv[i] = T.x_get[i];
@@ -392,8 +380,8 @@ __device__ __forceinline__ void chain_step(const Tile<NB, GATED>& T, const StepI
   load_weights(T, I1, W_next);
   // The loads stay here, a step ahead of their use.
   __builtin_amdgcn_sched_barrier(0);
-  chain_half<NB, GATED, F, 0>(xv, W, acc);
-  chain_half<NB, GATED, F, 1>(xv, W, acc);
+  chain_half<NB, F, 0>(xv, W, acc);
+  chain_half<NB, F, 1>(xv, W, acc);
   wave_sync();
 }
 
@@ -413,18 +401,15 @@ __device__ __forceinline__ void close_pass(typename Mfma<NB>::Acc& acc,
 
 // Step t, with the schedule of steps t .. t + 2 in hand; starts reading
 // step t + 3's (first used a step later, so its wait costs nothing).
-template <int NB, bool GATED, int F>
-__device__ __forceinline__ void run_step(const Tile<NB, GATED>& T, const Schedule<NB>& S, int t,
+template <int NB, int F>
+__device__ __forceinline__ void run_step(const Tile<NB>& T, const Schedule<NB>& S, int t,
                                          StepInfo<NB> (&I)[4], float4 (&G)[8],
-                                         const Weights<GATED, F>& W, Weights<GATED, F>& W_next,
-                                         typename Mfma<NB>::Acc (&acc)[GATED ? 2 : 1],
-                                         float (&total)[GATED ? 2 : 1][Mfma<NB>::kSlots]) {
+                                         const Weights<false, F>& W, Weights<false, F>& W_next,
+                                         typename Mfma<NB>::Acc& acc,
+                                         float (&total)[Mfma<NB>::kSlots]) {
   I[3] = step_info(S, t + 3);
-  chain_step<NB, GATED, F>(T, I[1], I[2], G, W, W_next, acc);
-  if (I[0].flags & kCloses) {
-#pragma unroll
-    for (int m = 0; m < (GATED ? 2 : 1); ++m) close_pass<NB>(acc[m], total[m]);
-  }
+  chain_step<NB, F>(T, I[1], I[2], G, W, W_next, acc);
+  if (I[0].flags & kCloses) close_pass<NB>(acc, total);
   I[0] = I[1];
   I[1] = I[2];
   I[2] = I[3];
@@ -432,16 +417,13 @@ __device__ __forceinline__ void run_step(const Tile<NB, GATED>& T, const Schedul
 
 // Grid: x = D-row tiles, y = groups of kTileWaves x D tokens, a wave's own
 // D tokens. Rows and tokens past the ends are read clamped and not stored.
-template <int NB, bool GATED, int F = kQ4_0>
+template <int NB, int F = kQ4_0>
 __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
-    const DevStep* __restrict__ step, QMatrix w, QMatrix up,
-    const float* __restrict__ x, int x_stride, uint32_t x_bytes, float* __restrict__ y,
-    int y_stride, const uint32_t* __restrict__ edits, int layer, uint32_t edit_stride,
-    const Schedule<NB> S) {
+    const DevStep* __restrict__ step, QMatrix w, const float* __restrict__ x, int x_stride,
+    uint32_t x_bytes, float* __restrict__ y, int y_stride, const Schedule<NB> S) {
   using M = Mfma<NB>;
   constexpr int D = M::kDim;
   constexpr int SL = M::kSlots;
-  constexpr int kMats = GATED ? 2 : 1;
   __shared__ float4 staged[kTileWaves][kXBuf];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tokens = (int)step->tokens;
@@ -450,7 +432,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
   if (token0 >= tokens) return;
   const int groups = w.cols >> 5;
 
-  Tile<NB, GATED> T;
+  Tile<NB> T;
   T.block = lane / D;
   const int row = min((int)blockIdx.x * D + lane % D, w.rows - 1);
   // The tile's member (a fused product over members placed apart): members
@@ -463,15 +445,11 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
                                             : w.rows;
   const uint32_t blocks = (uint32_t)member_rows * (uint32_t)groups;
   T.row_group0 = (uint32_t)(row - ((int)blockIdx.x * D - mr.row)) * (uint32_t)groups;
-  T.codes[0] = buffer_of(mr.codes, (uint32_t)code_bytes(F) * blocks);
-  T.scales[0] = buffer_of(mr.scales, 2u * (uint32_t)scale_halves(F) * blocks);
-  if (GATED) {
-    T.codes[kMats - 1] = buffer_of(up.codes, 16 * blocks);
-    T.scales[kMats - 1] = buffer_of(up.scales, 2 * blocks);
-  }
+  T.codes = buffer_of(mr.codes, (uint32_t)code_bytes(F) * blocks);
+  T.scales = buffer_of(mr.scales, 2u * (uint32_t)scale_halves(F) * blocks);
   T.x = buffer_of(x, x_bytes);
 #pragma unroll
-  for (int i = 0; i < Tile<NB, GATED>::kTokenRows; ++i) {
+  for (int i = 0; i < Tile<NB>::kTokenRows; ++i) {
     // line 8 i + lane / 8 is token (8 i + lane / 8) % D
     const int tok = min(token0 + (8 * i + (lane >> 3)) % D, tokens - 1);
     T.x_off[i] = 4u * ((uint32_t)tok * (uint32_t)x_stride + 4u * (uint32_t)(lane & 7));
@@ -479,15 +457,12 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
   T.x_put = staged[wave] + (lane >> 3) * kXLine + (lane & 7);
   T.x_get = staged[wave] + lane * kXLine;
 
-  typename M::Acc acc[kMats];
-  float total[kMats][SL];
+  typename M::Acc acc;
+  float total[SL];
 #pragma unroll
-  for (int m = 0; m < kMats; ++m) {
+  for (int i = 0; i < NB * SL; ++i) acc[i] = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NB * SL; ++i) acc[m][i] = 0.0f;
-#pragma unroll
-    for (int o = 0; o < SL; ++o) total[m][o] = 0.0f;
-  }
+  for (int o = 0; o < SL; ++o) total[o] = 0.0f;
 
   // Step 0 staged; step 1's inputs and step 0's weights in registers.
   StepInfo<NB> I[4];
@@ -498,33 +473,23 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
   load_inputs(T, I[0], G);
   stage_inputs(T, I[0], G);
   load_inputs(T, I[1], G);
-  Weights<GATED, F> W0, W1;
+  Weights<false, F> W0, W1;
   load_weights(T, I[0], W0);
   wave_sync();
   for (int t = 0; t < S.steps; t += 2) {
-    run_step<NB, GATED, F>(T, S, t, I, G, W0, W1, acc, total);
+    run_step<NB, F>(T, S, t, I, G, W0, W1, acc, total);
     if (t + 1 >= S.steps) break;
-    run_step<NB, GATED, F>(T, S, t + 1, I, G, W1, W0, acc, total);
+    run_step<NB, F>(T, S, t + 1, I, G, W1, W0, acc, total);
   }
 
   const int tok = token0 + lane % D;
   if (tok >= tokens) return;
   float* yrow = y + (size_t)tok * y_stride;
   const int row0 = blockIdx.x * D;
-  // A variants step: every row at the step's position, under its own table.
-  const uint32_t position = step->position + (step->variants ? 0u : (uint32_t)tok);
-  if (edits && step->variants) edits += (size_t)tok * edit_stride;
 #pragma unroll
   for (int o = 0; o < SL; ++o) {
     const int n = row0 + M::slot_row(lane, o);
-    if (n >= w.rows) continue;
-    if (!GATED) {
-      yrow[n] = total[0][o];
-    } else {
-      float v = gelu_tanh(total[0][o]) * total[kMats - 1][o];
-      if (edits) v = apply_edits(edits, layer, (uint32_t)n, position, v);
-      yrow[n] = v;
-    }
+    if (n < w.rows) yrow[n] = total[o];
   }
 }
 
@@ -667,12 +632,12 @@ __device__ __forceinline__ void load_pass_weights(const PassLane<GATED, F>& L, i
 template <bool GATED, int F>
 __device__ __forceinline__ void pass_products(const float4 (&xv)[8], const Weights<GATED, F>& W,
                                               typename Mfma<4>::Acc (&acc)[GATED ? 2 : 1]) {
-  if constexpr (GATED && F == kQ4_0) {
+  if constexpr (GATED) {
     chain_half_two<0>(xv, W, acc);
     chain_half_two<1>(xv, W, acc);
   } else {
-    chain_half<4, GATED, F, 0>(xv, W, acc);
-    chain_half<4, GATED, F, 1>(xv, W, acc);
+    chain_half<4, F, 0>(xv, W, acc[0]);
+    chain_half<4, F, 1>(xv, W, acc[0]);
   }
 }
 
@@ -946,6 +911,205 @@ __global__ __launch_bounds__(kPassWaves / HALVES * 64, 4 / HALVES) void pass_til
   }
 }
 
+// ---- gated products of many rows: a range at a time, weights shared --------
+// From a few hundred rows on (a prompt's 512-token step) the tiles fill the
+// chip and the fp32 matrix cores' own time is the bound; vector instructions
+// run beside none of it, so each one spent decoding or staging is time lost.
+// A workgroup of four waves owns D neurons' gate and up rows and 128 tokens,
+// each wave 32 of them, and chains the K ranges one after another. The
+// instruction's blocks are the two row blocks (and, at D = 16, two token
+// blocks) instead of ranges, so no block waits for a longer range (36 steps
+// at K = 1,152, where two ranges at a time take 40), an input line serves
+// gate and up, and the accumulators take half the registers: three (D = 32) or
+// four (D = 16) waves a SIMD instead of two. A group's weights are decoded
+// once into LDS for the four waves, and each wave's inputs go straight to its
+// LDS slot; both are double-buffered, step s + 1's fetched and decoded under
+// step s's products, with one barrier a step. A range opens on a product
+// with a zero addend, which is the chain's first fma.
+// 6,912 neurons over K = 1,152 took 215 us at 512 rows and 160 at 384 with a
+// wave a tile of two ranges; now 190 and 143 (86 TFLOP/s; the matrix cores
+// alone need 104 at 2.2 GHz, and 3.4 tiles a SIMD round up to 3.5).
+constexpr int kWideTokens = 32;  // a wave's tokens
+constexpr int kWideWaves = 4;
+constexpr int kWideGroups = 512;  // most groups of K
+
+template <int NB>
+__global__ __launch_bounds__(kWideWaves * 64, NB == 4 ? 4 : 3) void wide_gated_kernel(
+    const DevStep* __restrict__ step, QMatrix w, QMatrix up, const float* __restrict__ x,
+    uint32_t x_bytes, float* __restrict__ act, const uint32_t* __restrict__ edits, int layer,
+    uint32_t edit_stride) {
+  using M = Mfma<NB>;
+  constexpr int D = M::kDim, SL = M::kSlots, kRows = 2 * D, TB = NB / 2;
+  static_assert(TB * D == kWideTokens, "a wave's blocks hold its tokens");
+  __shared__ __align__(16) float4 weights[2][kRows * 8];
+  // Two arrays, so that a read of one waits for no load into the other.
+  __shared__ __align__(16) float4 inputs0[kWideWaves * kWideTokens * 8];
+  __shared__ __align__(16) float4 inputs1[kWideWaves * kWideTokens * 8];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int tokens = (int)step->tokens;
+  const int span0 = (int)blockIdx.y * kWideWaves * kWideTokens;
+  if (span0 >= tokens) return;  // the whole workgroup
+  const int token0 = span0 + wave * kWideTokens;
+  // A wave past the step's tokens decodes its share and waits with the rest.
+  const bool active = token0 < tokens;
+  const int groups = w.cols >> 5;
+
+  // This thread's row of the tile (gate rows, then up rows; rows past the end
+  // are read clamped and not stored) and its share of each group: code bytes
+  // 4 q .. 4 q + 3, both nibbles (D = 32) or one (D = 16).
+  constexpr int kThreadsRow = kWideWaves * 64 / kRows;
+  const int tile_row = t / kThreadsRow, part = t % kThreadsRow;
+  const int q = D == 32 ? part : part >> 1;
+  const int high = D == 32 ? 0 : part & 1;
+  const int row = min((int)blockIdx.x * D + tile_row % D, w.rows - 1);
+  const uint8_t* code_at =
+      (tile_row >= D ? up.codes : w.codes) + (size_t)row * groups * 16 + 4 * q;
+  const uint16_t* scale_at = (tile_row >= D ? up.scales : w.scales) + (size_t)row * groups;
+  struct Share {
+    uint32_t c;
+    uint16_t d;
+  };
+  auto load_share = [&](int g) {
+    return Share{*reinterpret_cast<const uint32_t*>(code_at + (size_t)g * 16), scale_at[g]};
+  };
+  // Row r's float4 f of a group at r * 8 + (f ^ (r % 8)), decoded as
+  // decode_half does.
+  auto put_share = [&](const Share& in, float4* dst) {
+    const float d = half_to_float(in.d);
+    float4* line = dst + tile_row * 8;
+    uint32_t kExp;
+    asm("v_mov_b32 %0, 0x64006400" : "=v"(kExp));
+    // At D = 16 the thread's nibble, brought to the low ones.
+    const uint32_t word = in.c >> (D == 16 ? 4 * high : 0);
+#pragma unroll
+    for (int h = 0; h < (D == 32 ? 2 : 1); ++h) {
+      const float scale = h == 0 ? d : 0.0625f * d;
+      const float bias = (h == 0 ? -1032.0f : -72.0f) * d;
+      const uint32_t mask = h == 0 ? 0x000F000Fu : 0x00F000F0u;
+      const half2v e = __builtin_bit_cast(half2v, (word & mask) | (kExp & ~mask));
+      const half2v o = __builtin_bit_cast(half2v, ((word >> 8) & mask) | (kExp & ~mask));
+      line[(4 * (D == 32 ? h : high) + q) ^ (tile_row & 7)] = make_float4(
+          __builtin_fmaf((float)e.x, scale, bias), __builtin_fmaf((float)o.x, scale, bias),
+          __builtin_fmaf((float)e.y, scale, bias), __builtin_fmaf((float)o.y, scale, bias));
+    }
+  };
+
+  // The wave's inputs of a group: token k's float4 f at k * 8 + (f ^ (k % 8)),
+  // loaded straight to LDS; instruction i is tokens 8 i .. 8 i + 7.
+  const __amdgpu_buffer_rsrc_t xr = buffer_of(x, x_bytes);
+  uint32_t x_off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int tok = min(token0 + 8 * i + (lane >> 3), tokens - 1);
+    x_off[i] = 4u * (uint32_t)tok * (uint32_t)w.cols + 16u * (uint32_t)((lane & 7) ^ (lane >> 3));
+  }
+  auto load_slot = [&](int g, float4* slot) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_to_lds(xr, slot + 64 * i, x_off[i], 128u * (uint32_t)g);
+  };
+
+  // Lane l: row block (l / D) % 2, token block l / (2 D), row or token l % D.
+  const int a_row = ((lane / D) & 1) * D + lane % D;
+  const int b_tok = ((lane / D) >> 1) * D + lane % D;
+  const uint32_t a_at = (uint32_t)(a_row * 8 * 16 + 16 * (a_row & 7));
+  const uint32_t b_at = (uint32_t)(b_tok * 8 * 16 + 16 * (b_tok & 7));
+
+  typename M::Acc acc, zero;
+  float total[NB * SL];
+#pragma unroll
+  for (int i = 0; i < NB * SL; ++i) acc[i] = 0.0f, zero[i] = 0.0f, total[i] = 0.0f;
+
+  float4* const slot0 = inputs0 + wave * kWideTokens * 8;
+  float4* const slot1 = inputs1 + wave * kWideTokens * 8;
+  load_slot(0, slot0);
+  Share held = load_share(0);
+  put_share(held, weights[0]);
+  held = load_share(min(1, groups - 1));
+  __syncthreads();
+  // The group after the open range's last; a range of fewer than 32 groups'
+  // K is one group or none. Whether the next group opens a range.
+  int range = 0, end = max(groups >> 5, 1);
+  bool opens = true;
+  // Quarter c of a group's operands: float4s 2 c and 2 c + 1 of the lane's
+  // lines, read a quarter ahead of its eight products.
+  auto read_quarter = [&](const float4* wp, const float4* xp, int c, float4 (&av)[2],
+                          float4 (&bv)[2]) {
+    const char* a_line = reinterpret_cast<const char*>(wp);
+    const char* b_line = reinterpret_cast<const char*>(xp);
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      av[f] = *reinterpret_cast<const float4*>(a_line + (a_at ^ (16u * (2 * c + f))));
+      bv[f] = *reinterpret_cast<const float4*>(b_line + (b_at ^ (16u * (2 * c + f))));
+    }
+  };
+  auto step_of = [&](int g, const float4* w_cur, float4* w_next, const float4* x_cur,
+                     float4* x_next) {
+    float4 av[2][2], bv[2][2];
+    if (active) {
+      read_quarter(w_cur, x_cur, 0, av[0], bv[0]);
+      read_quarter(w_cur, x_cur, 1, av[1], bv[1]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    put_share(held, w_next);
+    held = load_share(min(g + 2, groups - 1));
+    load_slot(min(g + 1, groups - 1), x_next);
+    __builtin_amdgcn_sched_barrier(0);
+    if (active) {
+      if (opens) {
+        acc = M::op(av[0][0].x, bv[0][0].x, zero);
+      } else {
+        acc = M::op(av[0][0].x, bv[0][0].x, acc);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          const float4 a = av[c & 1][f], b = bv[c & 1][f];
+          if (c > 0 || f > 0) acc = M::op(a.x, b.x, acc);
+          acc = M::op(a.y, b.y, acc);
+          acc = M::op(a.z, b.z, acc);
+          acc = M::op(a.w, b.w, acc);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (c < 2) read_quarter(w_cur, x_cur, c + 2, av[c & 1], bv[c & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (g + 1 == end) {
+#pragma unroll
+        for (int i = 0; i < NB * SL; ++i) total[i] = total[i] + acc[i];
+      }
+    }
+    opens = g + 1 == end;
+    if (opens) end = groups <= kRanges ? g + 2 : ((++range + 1) * groups) >> 5;
+    __syncthreads();
+  };
+  for (int g = 0; g < groups; g += 2) {
+    step_of(g, weights[0], weights[1], slot0, slot1);
+    if (g + 1 >= groups) break;
+    step_of(g + 1, weights[1], weights[0], slot1, slot0);
+  }
+
+  if (!active) return;
+#pragma unroll
+  for (int tb = 0; tb < TB; ++tb) {
+    const int tok = token0 + tb * D + lane % D;
+    if (tok >= tokens) continue;
+    float* out = act + (size_t)tok * w.rows;
+    // A variants step: every row at the step's position, under its own table.
+    const uint32_t position = step->position + (step->variants ? 0u : (uint32_t)tok);
+    const uint32_t* table = edits && step->variants ? edits + (size_t)tok * edit_stride : edits;
+#pragma unroll
+    for (int o = 0; o < SL; ++o) {
+      const int n = (int)blockIdx.x * D + M::slot_row(lane, o);
+      if (n >= w.rows) continue;
+      float v = gelu_tanh(total[SL * 2 * tb + o]) * total[SL * (2 * tb + 1) + o];
+      if (table) v = apply_edits(table, layer, (uint32_t)n, position, v);
+      out[n] = v;
+    }
+  }
+}
+
 // The passes: ranges sorted by length, longest first, four a pass (each
 // half's own ranges when a tile is split in halves).
 PassOrder pass_order(int groups, int halves) {
@@ -1020,10 +1184,9 @@ hipError_t launch_pass_tiles(hipStream_t s, const DevStep* step, QMatrix w, QMat
   return hipGetLastError();
 }
 
-template <int NB, bool GATED, int F = kQ4_0>
-hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, QMatrix up,
-                         const float* x, int x_stride, float* y, int y_stride, int max_tokens,
-                         const uint32_t* edits, int layer, uint32_t edit_stride = 0) {
+template <int NB, int F = kQ4_0>
+hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, const float* x,
+                         int x_stride, float* y, int y_stride, int max_tokens) {
   constexpr int D = Mfma<NB>::kDim;
   const int groups = w.cols >> 5;
   const uint64_t x_bytes = 4ull * (uint64_t)x_stride * (uint64_t)max_tokens;
@@ -1035,8 +1198,41 @@ hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, QMatrix 
   }
   const int token_span = kTileWaves * D;
   const dim3 grid((w.rows + D - 1) / D, (max_tokens + token_span - 1) / token_span);
-  hipLaunchKernelGGL((gemm_ranges<NB, GATED, F>), grid, dim3(kTileWaves * 64), 0, s, step, w, up,
-                     x, x_stride, (uint32_t)x_bytes, y, y_stride, edits, layer, edit_stride, S);
+  hipLaunchKernelGGL((gemm_ranges<NB, F>), grid, dim3(kTileWaves * 64), 0, s, step, w, x, x_stride,
+                     (uint32_t)x_bytes, y, y_stride, S);
+  return hipGetLastError();
+}
+
+// The gated product a pass a wave took 92 us at 192 rows and 120 at 256
+// (6,912 neurons, K = 1,152), its wide tiles 97 and 104: they fill their
+// 128-token spans a step at a time.
+constexpr int kGatedPassRows = 208;
+
+hipError_t launch_wide(hipStream_t s, const DevStep* step, QMatrix gate, QMatrix up,
+                       const float* x, float* act, int max_tokens, const uint32_t* edits,
+                       int layer, uint32_t edit_stride) {
+  const int groups = gate.cols >> 5;
+  const uint64_t x_bytes = 4ull * (uint64_t)gate.cols * (uint64_t)max_tokens;
+  const uint64_t codes = 16ull * (uint64_t)gate.rows * (uint64_t)groups;
+  if (groups < 1 || groups > kWideGroups || x_bytes >= (1ull << 31) || codes >= (1ull << 31))
+    return hipErrorInvalidValue;
+  const int span = kWideWaves * kWideTokens;
+  const int spans = (max_tokens + span - 1) / span;
+  auto launch = [&](auto kernel, int neurons) {
+    hipLaunchKernelGGL(kernel, dim3((gate.rows + neurons - 1) / neurons, spans),
+                       dim3(kWideWaves * 64), 0, s, step, gate, up, x, (uint32_t)x_bytes, act,
+                       edits, layer, edit_stride);
+  };
+  // Tiles of 32 neurons do a little better (half the LDS reads a product)
+  // while all their workgroups fit on the 256 CUs at once, three each; past
+  // that the last round is nearly empty, and tiles of 16, four workgroups a
+  // CU, even it out: 198 and 190 us at 512 rows of 6,912 neurons, 143 and 151
+  // at 384, 104 and 113 at 256.
+  if (((gate.rows + 31) / 32) * spans <= 3 * 256) {
+    launch(wide_gated_kernel<2>, 32);
+  } else {
+    launch(wide_gated_kernel<4>, 16);
+  }
   return hipGetLastError();
 }
 
@@ -1047,9 +1243,12 @@ hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, QMatrix 
 // decoded weights are shared by 32 tokens there, by 16 here). A matrix of
 // thousands of tiles (the vocabulary's) fills the chip a wave a tile from 17
 // rows on.
-bool pass_tiles(const QMatrix& w, int max_tokens) {
-  const int most = w.rows < 512 * Mfma<4>::kDim ? kSplitRows : Mfma<4>::kDim;
-  return max_tokens <= most && (w.cols >> 5) >= kRanges;
+bool pass_tiles(const QMatrix& w, int max_tokens, int x_stride) {
+  const int groups = w.cols >> 5;
+  // Past 16 rows, only what gemm_ranges would take as well.
+  const bool many = w.rows < 512 * Mfma<4>::kDim && groups <= kWideGroups &&
+                    4ull * (uint64_t)x_stride * (uint64_t)max_tokens < kPastEnd;
+  return max_tokens <= (many ? kSplitRows : Mfma<4>::kDim) && groups >= kRanges;
 }
 
 }  // namespace
@@ -1071,7 +1270,7 @@ hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
   // 32 x 32 tiles waste half their columns on 16 tokens or fewer.
   const bool wide = (size_t)w.rows * (size_t)max_tokens >= (size_t)768 * 1024 &&
                     max_tokens > Mfma<4>::kDim;
-  if (pass_tiles(w, max_tokens)) {
+  if (pass_tiles(w, max_tokens, x_stride)) {
     switch (w.format) {
       case kQ4_0:
         // Thousands of tiles (a vocabulary's head) go a pair to a wave: half
@@ -1094,22 +1293,16 @@ hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
   switch (w.format) {
     case kQ4_0:
       if (wide)
-        return launch_ranges<2, false>(s, step, w, w, x, x_stride, y, y_stride, max_tokens,
-                                       nullptr, 0);
-      return launch_ranges<4, false>(s, step, w, w, x, x_stride, y, y_stride, max_tokens, nullptr,
-                                     0);
+        return launch_ranges<2>(s, step, w, x, x_stride, y, y_stride, max_tokens);
+      return launch_ranges<4>(s, step, w, x, x_stride, y, y_stride, max_tokens);
     case kQ4_1:
       if (wide)
-        return launch_ranges<2, false, kQ4_1>(s, step, w, w, x, x_stride, y, y_stride,
-                                              max_tokens, nullptr, 0);
-      return launch_ranges<4, false, kQ4_1>(s, step, w, w, x, x_stride, y, y_stride, max_tokens,
-                                            nullptr, 0);
+        return launch_ranges<2, kQ4_1>(s, step, w, x, x_stride, y, y_stride, max_tokens);
+      return launch_ranges<4, kQ4_1>(s, step, w, x, x_stride, y, y_stride, max_tokens);
     case kQ8_0:
       if (wide)
-        return launch_ranges<2, false, kQ8_0>(s, step, w, w, x, x_stride, y, y_stride,
-                                              max_tokens, nullptr, 0);
-      return launch_ranges<4, false, kQ8_0>(s, step, w, w, x, x_stride, y, y_stride, max_tokens,
-                                            nullptr, 0);
+        return launch_ranges<2, kQ8_0>(s, step, w, x, x_stride, y, y_stride, max_tokens);
+      return launch_ranges<4, kQ8_0>(s, step, w, x, x_stride, y, y_stride, max_tokens);
     default:
       return hipErrorInvalidValue;
   }
@@ -1119,7 +1312,7 @@ hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
 // 72 tiles of 216 groups would keep one workgroup of 8 waves on each of 72
 // CUs, two chains a SIMD; split, 144 workgroups of 4 waves take one a SIMD.
 bool gemv_splits(const QMatrix& w, int max_tokens) {
-  return max_tokens > 1 && pass_tiles(w, max_tokens) && (w.cols >> 5) >= 4 * kRanges &&
+  return max_tokens > 1 && pass_tiles(w, max_tokens, w.cols) && (w.cols >> 5) >= 4 * kRanges &&
          w.rows <= 256 * Mfma<4>::kDim && !has_members(w);
 }
 
@@ -1154,12 +1347,11 @@ hipError_t launch_gated(hipStream_t s, const DevStep* step, QMatrix gate,
     in.x = x;
     return launch_gated_decode(s, step, gate, up, in, 0, act, edits, layer);
   }
-  if (pass_tiles(gate, max_tokens)) {
+  if (pass_tiles(gate, max_tokens, gate.cols) && max_tokens <= kGatedPassRows) {
     return launch_pass_tiles<kGatedKind, kQ4_0>(s, step, gate, up, x, gate.cols, act, gate.rows,
                                           max_tokens, edits, layer, edit_stride);
   }
-  return launch_ranges<2, true>(s, step, gate, up, x, gate.cols, act, gate.rows, max_tokens, edits,
-                               layer, edit_stride);
+  return launch_wide(s, step, gate, up, x, act, max_tokens, edits, layer, edit_stride);
 }
 
 }  // namespace frz

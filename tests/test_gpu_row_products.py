@@ -41,10 +41,15 @@ def test_row_products_bit_exact(device, fmt, rows, cols, tokens):
     _check_rows(dy.numpy(), lambda t: orc.gemv_format(fmt, w, rows, cols, x[t]), tokens)
 
 
-@pytest.mark.parametrize("rows,tokens", [(6912, 17), (1000, 48), (96, 256), (96, 257), (100, 512)])
-def test_gated_rows_bit_exact(device, rows, tokens):
+# Past 208 rows the wide tiles: of 32 neurons while their workgroups fit on the
+# chip at once, else of 16; K of fewer groups than ranges goes there at any rows.
+@pytest.mark.parametrize("rows,tokens,cols", [
+    (6912, 17, 1152), (1000, 48, 1152), (96, 256, 1152), (96, 257, 1152), (100, 512, 1152),
+    (95, 208, 1152), (1000, 209, 1152), (6900, 510, 1152), (6900, 385, 1056), (33, 300, 1056),
+    (50, 2, 32), (40, 9, 96), (70, 161, 992), (70, 225, 1024)])
+def test_gated_rows_bit_exact(device, rows, tokens, cols):
     rng = np.random.default_rng(rows + tokens)
-    cols, layers, layer, position = 1152, 2, 1, 30
+    layers, layer, position = 2, 1, 30
     g, u = q4_blocks(rng, rows, cols), q4_blocks(rng, rows, cols)
     x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
     # Pins that start and end inside the step, at the first and last neurons.
