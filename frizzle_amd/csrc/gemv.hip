@@ -525,9 +525,8 @@ bool build_schedule(int groups, Schedule<NB>& S) {
   return t > 0;
 }
 
-// ---- steps of up to a few hundred rows: a pass a wave ----------------------
-// A step of few rows (a batch of variants, a chat message, a prompt's last
-// rows) makes one 16 x 16 tile per 16 output rows and 16 tokens. With a wave
+// ---- a pass a wave ----------------------------------------------------------
+// A step of several rows (a batch of variants, a chat message, a prompt) makes one 16 x 16 tile per 16 output rows and 16 tokens. With a wave
 // a tile (gemm_ranges) its 32 ranges are one serial chain, which is all the
 // time there is until the tiles fill the chip: 55 us for gate and up and 51
 // for down at any 17 to 128 tokens. Here a workgroup takes a tile and its eight
@@ -1236,19 +1235,18 @@ hipError_t launch_wide(hipStream_t s, const DevStep* step, QMatrix gate, QMatrix
   return hipGetLastError();
 }
 
-// A step over K of 32 groups or more takes a pass a wave up to kSplitRows
-// rows, where the tiles of a wave each (gemm_ranges) catch up: a layer's
-// products took, a wave a tile then a pass a wave, 142 then 56 us at 32
-// rows, 153 then 125 at 128, 230 then 209 at 256, 378 then 389 at 512 (the
-// decoded weights are shared by 32 tokens there, by 16 here). A matrix of
-// thousands of tiles (the vocabulary's) fills the chip a wave a tile from 17
-// rows on.
+// A step over K of 32 groups or more takes a pass a wave, whose workgroups are
+// small enough to fill the chip at every row count and to even out its last
+// round. gemm_ranges, a wave a tile, took for Q/K/V, O and down 25, 18 and 90
+// us at 288 rows and 38, 24 and 121 at 512; a pass a wave 23, 16 and 75, and
+// 34, 23 and 112. A matrix of thousands of tiles (the vocabulary's) fills the
+// chip a wave a tile from 17 rows on.
 bool pass_tiles(const QMatrix& w, int max_tokens, int x_stride) {
   const int groups = w.cols >> 5;
   // Past 16 rows, only what gemm_ranges would take as well.
   const bool many = w.rows < 512 * Mfma<4>::kDim && groups <= kWideGroups &&
                     4ull * (uint64_t)x_stride * (uint64_t)max_tokens < kPastEnd;
-  return max_tokens <= (many ? kSplitRows : Mfma<4>::kDim) && groups >= kRanges;
+  return (many || max_tokens <= Mfma<4>::kDim) && groups >= kRanges;
 }
 
 }  // namespace
@@ -1310,10 +1308,12 @@ hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
 
 // Splitting pays where a tile's chains are long and the tiles few: down's
 // 72 tiles of 216 groups would keep one workgroup of 8 waves on each of 72
-// CUs, two chains a SIMD; split, 144 workgroups of 4 waves take one a SIMD.
+// CUs, two chains a SIMD; split, 144 workgroups of 4 waves take one a SIMD
+// (16 rows: 15.8 -> 10.0 us). A second token tile makes as many workgroups
+// (17 to 32 rows: 16.0 split, 14.5 whole).
 bool gemv_splits(const QMatrix& w, int max_tokens) {
-  return max_tokens > 1 && pass_tiles(w, max_tokens, w.cols) && (w.cols >> 5) >= 4 * kRanges &&
-         w.rows <= 256 * Mfma<4>::kDim && !has_members(w);
+  return max_tokens > 1 && max_tokens <= kSplitRows && pass_tiles(w, max_tokens, w.cols) &&
+         (w.cols >> 5) >= 4 * kRanges && w.rows <= 256 * Mfma<4>::kDim && !has_members(w);
 }
 
 hipError_t launch_gemv_split(hipStream_t s, const DevStep* step, QMatrix w, const float* x,

@@ -10,7 +10,7 @@ namespace frz {
 
 constexpr int kRanges = 32;        // a row's K-ranges (matmul.h:88-97)
 constexpr int kSplitParts = kRanges / 2;  // range sums a split product leaves apart
-constexpr int kSplitRows = 256;           // most rows a split product takes
+constexpr int kSplitRows = 16;            // most rows a split product takes
 constexpr int kChunkKeys = 64;     // attention chunk (attention.wgsl:60)
 constexpr int kTileKeys = 8;       // attention tile at d = 256
 constexpr int kCandidates = 64;    // top-k kept (residency/plan.h:195)
