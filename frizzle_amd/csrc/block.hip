@@ -283,6 +283,23 @@ __global__ __launch_bounds__(256) void capture_weights_kernel(const DevStep* __r
     w[i] = (uint32_t)i < read ? exp2f_fixed(w[i] - m) / l : 0.0f;
 }
 
+// ---- a prefix's cache rows into each variant's caches -------------------------
+// Grid: x = 256 pieces of 16 bytes, y = keys or values, z = the copy. The
+// prefix's rows come from L2 after the first copy's reads, so the writes bound
+// it: 299 rows of a layer for 16 variants (4.9 MB) take 4 us, where a copy a
+// variant and cache of the whole ring had been 32 copies of 3 us.
+__global__ __launch_bounds__(256) void spread_rows_kernel(const uint4* __restrict__ keys,
+                                                          const uint4* __restrict__ values,
+                                                          uint4* __restrict__ key_copies,
+                                                          uint4* __restrict__ value_copies,
+                                                          size_t pieces, size_t stride) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= pieces) return;
+  const uint4* src = blockIdx.y ? values : keys;
+  uint4* dst = (blockIdx.y ? value_copies : key_copies) + blockIdx.z * stride;
+  dst[i] = src[i];
+}
+
 // ---- pins (edit.wgsl:55-76) ----------------------------------------------------
 __global__ __launch_bounds__(64) void edit_kernel(const DevStep* __restrict__ step,
                                                   const uint32_t* __restrict__ table,
@@ -345,6 +362,19 @@ hipError_t launch_capture_weights(hipStream_t s, const DevStep* step, float* wei
   if (keys <= 0 || query_heads <= 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(capture_weights_kernel, dim3(query_heads), dim3(256), 0, s, step, weights,
                      stats, keys);
+  return hipGetLastError();
+}
+
+hipError_t launch_spread_rows(hipStream_t s, const uint16_t* keys, const uint16_t* values,
+                              uint16_t* key_copies, uint16_t* value_copies, size_t elems,
+                              size_t stride, int copies) {
+  if (elems == 0) return hipSuccess;
+  if (elems % 8 != 0 || stride % 8 != 0 || copies < 1) return hipErrorInvalidValue;
+  const size_t pieces = elems / 8;
+  hipLaunchKernelGGL(spread_rows_kernel, dim3((unsigned)((pieces + 255) / 256), 2, copies),
+                     dim3(256), 0, s, reinterpret_cast<const uint4*>(keys),
+                     reinterpret_cast<const uint4*>(values), reinterpret_cast<uint4*>(key_copies),
+                     reinterpret_cast<uint4*>(value_copies), pieces, stride / 8);
   return hipGetLastError();
 }
 

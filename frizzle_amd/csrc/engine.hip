@@ -1945,21 +1945,17 @@ int frz_generate_variants(frz_model* m, const uint32_t* prompt, uint32_t prompt_
   frz_model::Variants& V = m->variants;
   V.capture = residuals_out != nullptr;
   hipStream_t s = m->dev->stream;
-  // Every variant's caches start as the prefix's.
+  // Every variant's caches start as the prefix's: the rows of positions 0 to
+  // origin - 1, or the whole ring once they have been round it. A slot past
+  // them is written before it is read as a live key.
   const size_t kvw = (size_t)c.kv_heads * c.head_dim;
   for (int l = 0; l < c.layers; ++l) {
     const Layer& L = m->layers[l];
-    const size_t bytes = (size_t)L.slots * kvw * 2, elems = (size_t)L.slots * kvw;
-    for (uint32_t v = 0; v < variants; ++v) {
-      if (int rc = check_hip(hipMemcpyAsync(V.kcache[l] + v * elems, L.kcache, bytes,
-                                            hipMemcpyDeviceToDevice, s),
-                             "variant keys"))
-        return rc;
-      if (int rc = check_hip(hipMemcpyAsync(V.vcache[l] + v * elems, L.vcache, bytes,
-                                            hipMemcpyDeviceToDevice, s),
-                             "variant values"))
-        return rc;
-    }
+    const size_t rows = std::min<size_t>((size_t)L.slots, origin);
+    if (int rc = check_hip(launch_spread_rows(s, L.kcache, L.vcache, V.kcache[l], V.vcache[l],
+                                              rows * kvw, (size_t)L.slots * kvw, (int)variants),
+                           "variant caches"))
+      return rc;
   }
   std::vector<uint32_t> tables((size_t)variants * V.edit_stride, 0);
   for (uint32_t v = 0; v < variants; ++v)

@@ -404,6 +404,12 @@ constexpr int kMaxFoldChunks = 224;  // chunk states of the static decode worksp
 // partial chunk a window straddles (the fold stages them in segments).
 constexpr int kMaxContextChunks = 32768 / kChunkKeys + 1;
 
+// The first `elems` F16 values of a layer's keys and values (whole 16-byte
+// pieces) into `copies` caches, stride values apart.
+hipError_t launch_spread_rows(hipStream_t s, const uint16_t* keys, const uint16_t* values,
+                              uint16_t* key_copies, uint16_t* value_copies, size_t elems,
+                              size_t stride, int copies);
+
 // The capture store's copies at the step that ends the prompt: the last row
 // of src (rows row_stride words apart) into dst, word for word
 // (capture.wgsl); and the last row's scores turned into attention weights

@@ -152,3 +152,19 @@ def test_variants_refusals(device):
             model.handle, prompt.ctypes.data, prompt.size, 1, bad.ctypes.data, bad.size,
             ctypes.byref(s), 4, None, 0, out.ctypes.data, drawn.ctypes.data, None))
     model.close()
+
+
+def test_variants_start_from_the_prefix_rows_alone(device):
+    # A prompt that goes round the sliding layers' rings, then a shorter one
+    # whose variants' caches keep the longer one's rows past their prefix, then
+    # one of a single token (no prefix): each reply is the one made alone.
+    cfg = small_config()
+    model, _ = build_pair(device, cfg, seed=53)
+    rng = np.random.default_rng(54)
+    variants = seeded_variants(cfg, rng, 5)
+    for n in (cfg.local_slots + 37, cfg.local_slots, 77, 1):
+        prompt = rng.integers(0, cfg.vocab, n).astype(np.uint32)
+        got = model.generate_variants(prompt, variants, max_tokens=6)
+        for v, edits in enumerate(variants):
+            assert np.array_equal(got[v], model.generate(prompt, edits, max_tokens=6)), (n, v)
+    model.close()
