@@ -75,6 +75,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(
   const int row = a.last_token ? (int)step->tokens - 1 : (int)blockIdx.x;
   const int vec4s = a.width / 4;
   const size_t base = (size_t)row * a.width;
+  const size_t from = a.hidden_words ? (size_t)a.hidden_words[row] : base;
   const float n = (float)a.width;
   const int i = threadIdx.x;
   float4 x[kNormMaxVec4], y[kNormMaxVec4], pg[kNormMaxVec4], g[kNormMaxVec4];
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(
   for (int k = 0; k < kNormMaxVec4; ++k) {
     const int q = i + k * kNormThreads;
     if (k < per && q < vec4s) {
-      x[k] = ld4(a.hidden + base + 4 * q);
+      x[k] = ld4(a.hidden + from + 4 * q);
       g[k] = ld4(a.gain + 4 * q);
       if (a.post_gain) {
         y[k] = ld4(a.output + base + 4 * q);
@@ -325,7 +326,9 @@ __global__ __launch_bounds__(64) void edit_kernel(const DevStep* __restrict__ st
 
 hipError_t launch_norm(hipStream_t s, const DevStep* step, const NormArgs& a,
                        int max_tokens) {
-  if (a.width % 4 != 0 || a.width > 4 * kNormThreads * kNormMaxVec4) return hipErrorInvalidValue;
+  if (a.width % 4 != 0 || a.width > 4 * kNormThreads * kNormMaxVec4 ||
+      (a.hidden_words && a.post_gain))
+    return hipErrorInvalidValue;
   hipLaunchKernelGGL(norm_kernel, dim3(a.last_token ? 1 : max_tokens), dim3(kNormThreads), 0, s,
                      step, a);
   return hipGetLastError();

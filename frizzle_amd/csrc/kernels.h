@@ -275,6 +275,8 @@ struct NormArgs {
   // prefill products' inputs, plane_index order).
   uint16_t* normed_hi = nullptr;
   uint16_t* normed_lo = nullptr;
+  // Not null (no add): row r's hidden starts at hidden + hidden_words[r].
+  const uint32_t* hidden_words = nullptr;
 };
 hipError_t launch_norm(hipStream_t s, const DevStep* step, const NormArgs& a,
                        int max_tokens);
@@ -432,6 +434,10 @@ hipError_t launch_edit(hipStream_t s, const DevStep* step,
 size_t topk_scratch_words(int count);
 hipError_t launch_topk(hipStream_t s, const float* logits, int count,
                        uint32_t* scratch, uint32_t* candidates);
+// The same for `rows` rows of logits (scratch a row's words each), row r's
+// candidates at dst + at[r] (at in device memory).
+hipError_t launch_topk_rows(hipStream_t s, const float* logits, int count, int rows,
+                            uint32_t* scratch, uint32_t* dst, const uint32_t* at);
 // The top-64 as above, then the draw (as launch_draw) and, when `advance`,
 // the fed step's advance (as launch_advance), the last two in the final
 // selection kernel.

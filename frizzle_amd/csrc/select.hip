@@ -164,6 +164,15 @@ __global__ __launch_bounds__(64 * kMergeWaves) void topk_merge_kernel(const uint
   if (threadIdx.x < 64) store_entry(out, blockIdx.x * kCandidates + threadIdx.x, top);
 }
 
+// The last merge of row y's lists, into dst + at[y].
+__global__ __launch_bounds__(64 * kMergeWaves) void topk_rows_kernel(
+    const uint32_t* __restrict__ in, int lists, uint32_t* __restrict__ dst,
+    const uint32_t* __restrict__ at, size_t stride) {
+  __shared__ uint64_t shared[kMergeWaves][64];
+  const uint64_t top = merge_lists(in + blockIdx.y * stride, lists, shared);
+  if (threadIdx.x < 64) store_entry(dst + at[blockIdx.y], threadIdx.x, top);
+}
+
 // The high word of a * b from 16-bit halves (draw.wgsl:34-45).
 __device__ __forceinline__ uint32_t mulhi16(uint32_t a, uint32_t b) {
   const uint32_t a0 = a & 0xFFFFu, a1 = a >> 16, b0 = b & 0xFFFFu, b1 = b >> 16;
@@ -363,6 +372,16 @@ hipError_t launch_topk(hipStream_t s, const float* logits, int count,
                        candidates, (size_t)0);
     return hipGetLastError();
   });
+}
+
+hipError_t launch_topk_rows(hipStream_t s, const float* logits, int count, int rows,
+                            uint32_t* scratch, uint32_t* dst, const uint32_t* at) {
+  return select_passes(
+      s, logits, count, rows, scratch, [&](const uint32_t* in, int lists, size_t stride) {
+        hipLaunchKernelGGL(topk_rows_kernel, dim3(1, rows), dim3(64 * kMergeWaves), 0, s, in, lists,
+                           dst, at, stride);
+        return hipGetLastError();
+      });
 }
 
 hipError_t launch_select(hipStream_t s, DevStep* step, const float* logits, int count,

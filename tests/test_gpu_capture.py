@@ -122,3 +122,19 @@ def test_readouts_see_the_residual_where_each_layer_leaves_it(device):
     assert np.array_equal(readout(plain, 0), readout(pinned, 0))
     assert not np.array_equal(readout(plain, 1), readout(pinned, 1))
     model.close()
+
+
+# The readouts run in batches of 16 layers: one batch short, whole, and whole
+# with one or several rows after it.
+@pytest.mark.parametrize("layers", [1, 12, 17, 18, 20])
+def test_readouts_in_batches_are_the_oracles(device, layers):
+    cfg = small_config(layers=layers, vocab=1100)
+    model, oracle = build_pair(device, cfg, seed=70 + layers)
+    prompt = np.random.default_rng(layers).integers(0, cfg.vocab, 5).astype(np.uint32)
+    model.set_capture(True)
+    model.generate(prompt, (), max_tokens=0)
+    store, layout = model.capture()
+    o = oracle_capture(oracle, cfg, prompt, placed(cfg, [], len(prompt) - 1))
+    assert_store_is_oracles(store, layout, o, f"{layers} layers")
+    o.close()
+    model.close()
