@@ -25,12 +25,15 @@
 // 107 MB a layer, 2.8 GB in all.
 //
 // Tiles: a workgroup of eight waves (two a SIMD, so that one wave's
-// products run while the other waits) owns 128 output rows x 256 tokens and
-// steps K one 32-weight block at a time. Wave w computes all 128 rows for
-// tokens 32 w .. 32 w + 31 (four 32 x 32 accumulators): the weights, which
-// all eight waves read, pass through LDS (double-buffered), moved there by
-// waves 0-3; each wave's token fragments, which only it reads, go straight
-// into its registers. Loads run ahead and are copied as they are (no VALU). The
+// products run while the other waits) owns 128 output rows (64 in a step of
+// one token tile) x 256 tokens and steps K one 32-weight block at a time.
+// Wave w computes all its rows for tokens 32 w .. 32 w + 31 (four or two
+// 32 x 32 accumulators): the weights, which all eight waves read, pass
+// through LDS (double-buffered), a piece moved there by each wave; each
+// wave's token fragments, which only it reads, go straight into its
+// registers. Loads run ahead and are copied as they are (no VALU), and the
+// K loop's waits count exactly them: with an exit inside its unrolled turn
+// every turn had waited for loads just asked for. The
 // instruction takes the tokens as its A operand and the weights as B, so
 // that each output register's lanes are 32 consecutive rows of one token.
 // For the gated product, row blocks 0 and 1 are 64 neurons' gate rows and
@@ -230,21 +233,26 @@ __device__ __forceinline__ float gelu_fast(float g) {
   return g * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-// A wave's share of one K block (two steps of 16 k): its weight block's
-// fragments [step][hi, lo] (waves 0-3), staged in LDS for the workgroup, and
-// its token block's [step][hi, lo], which only it reads.
-struct WeightLoad2 {
-  uint4 w[2][2];
-};
+// A wave's token block of one K block (two steps of 16 k), which only it
+// reads.
 struct TokenLoad {
-  uint4 x[2][2];
+  uint4 x[2][2];  // [step][hi, lo]
 };
 
-template <bool GATED>
-__global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(const DevStep* __restrict__ step,
-                                                                Bf16Gemm g) {
+// RB: the row blocks a workgroup takes of a tile's four: all, or half (gated:
+// 32 neurons' gate and up blocks; else two neighbouring blocks).
+template <bool GATED, int RB>
+__global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(
+    const DevStep* __restrict__ step, Bf16Gemm g) {
+  constexpr int kSub = 4 / RB;
+  // A K block's weights are 4 RB pieces of 1 KB, moved to LDS by the eight
+  // waves alike; blocks of weights and of tokens in flight in registers.
+  constexpr int kPieces = RB / 2, kW = 4, kX = RB == 4 ? 2 : 4;
+  struct WeightLoad2 {
+    uint4 w[kPieces];
+  };
   // The weights of one K block: [step][row block][hi, lo][lane].
-  __shared__ uint4 stage[2][2][4][2][64];
+  __shared__ uint4 stage[2][2][RB][2][64];
   const int tokens = (int)step->tokens;
   // Workgroups go to the eight XCDs in turn (linear id mod 8); the tile
   // order gives each XCD a contiguous run of tiles, so that the token tiles
@@ -253,7 +261,9 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(const DevSte
   const int xcd = wid & 7, per = total >> 3, extra = total & 7;
   const int tile = xcd * per + min(xcd, extra) + (wid >> 3);
   const int tt = tile % g.token_tiles, rest = tile / g.token_tiles;
-  const int z = rest % g.splits, rt = rest / g.splits;
+  const int z = rest % g.splits, rt = rest / g.splits / kSub, sub = rest / g.splits % kSub;
+  // Block i of the workgroup's RB among the tile's four.
+  auto tile_block = [&](int i) { return RB == 4 ? i : GATED ? sub + 2 * i : 2 * sub + i; };
   const int n0 = tt * kTileTokens;
   if (n0 >= tokens) return;  // the whole workgroup: past the step's rows
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -264,9 +274,9 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(const DevSte
   // acc[row block][token block of the wave], transposed: the instruction
   // takes the tokens as its A operand and the weights as B, so a lane holds
   // one output row (lane % 32) for 16 tokens.
-  f32x16 acc[4];
+  f32x16 acc[RB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < RB; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
 
@@ -275,31 +285,33 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(const DevSte
   if (kb0 >= kb1) {
     if (!GATED) {
       float* y = g.y + (size_t)z * g.part_stride;
-      for (int i = tid; i < kTileRows * kTileTokens; i += kGemmThreads) {
-        const int o = rt * kTileRows + (i % kTileRows), t = n0 + i / kTileRows;
+      constexpr int kRows = 32 * RB;
+      for (int i = tid; i < kRows * kTileTokens; i += kGemmThreads) {
+        const int o = rt * kTileRows + sub * kRows + (i % kRows), t = n0 + i / kRows;
         if (o < g.rows && t < tokens) y[(size_t)t * g.ldy + o] = 0.0f;
       }
     }
     return;
   }
-  // Wave w < 4 moves weight block w of the row tile into LDS; wave w reads
-  // its token block w of the tile (the last block with rows, for blocks
-  // past them) straight into registers. Every fragment is a 1 KB run of its
-  // planes, 16 bytes a lane.
-  const bool mover = wave < 4;  // uniform over the wave
-  const uint4* wsrc = g.w + fragment_at(rt, steps, 0, wave & 3, 0) + lane;
+  // Wave w moves its pieces of the workgroup's weights into LDS and reads its
+  // token block w of the tile (the last block with rows, for blocks past
+  // them, whose products it leaves out) straight into registers. Every
+  // fragment is a 1 KB run of its planes, 16 bytes a lane.
+  const bool active = n0 + 32 * wave < tokens;  // uniform over the wave
+  const uint4* wsrc[kPieces];
+#pragma unroll
+  for (int j = 0; j < kPieces; ++j) {
+    const int piece = wave * kPieces + j;  // [step][row block][hi, lo]
+    wsrc[j] = g.w + fragment_at(rt, steps, piece / (2 * RB), tile_block(piece / 2 % RB), piece % 2) +
+              lane;
+  }
   const int last_tb = (tokens - 1) >> 5;
   const size_t x_at = plane_index(32 * min(n0 / 32 + wave, last_tb), 0, g.ldx) + 8 * lane;
   auto load_w = [&](int kb) {
     WeightLoad2 r;
-    if (mover) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const size_t s = 2 * (size_t)kb + u;
-        r.w[u][0] = load_global4(wsrc + s * (kStepBytes / 16));
-        r.w[u][1] = load_global4(wsrc + s * (kStepBytes / 16) + 64);
-      }
-    }
+    for (int j = 0; j < kPieces; ++j)
+      r.w[j] = load_global4(wsrc[j] + 2 * (size_t)kb * (kStepBytes / 16));
     return r;
   };
   auto load_x = [&](int kb) {
@@ -312,70 +324,71 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(const DevSte
     }
     return r;
   };
-  auto put = [&](uint4 (&st)[2][4][2][64], const WeightLoad2& r) {
+  auto put = [&](uint4 (&st)[2][RB][2][64], const WeightLoad2& r) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        if (mover) st[u][wave][p][lane] = r.w[u][p];
-      }
+    for (int j = 0; j < kPieces; ++j) {
+      const int piece = wave * kPieces + j;
+      (&st[0][0][0][0])[piece * 64 + lane] = r.w[j];
+    }
   };
-  auto compute = [&](const uint4 (&st)[2][4][2][64], const TokenLoad& r) {
+  auto compute = [&](const uint4 (&st)[2][RB][2][64], const TokenLoad& r) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      bf16x8 wh[4], wl[4];
+      bf16x8 wh[RB], wl[RB];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < RB; ++i) {
         wh[i] = as_bf16x8(st[u][i][0][lane]);
         wl[i] = as_bf16x8(st[u][i][1][lane]);
       }
       const bf16x8 xh = as_bf16x8(r.x[u][0]), xl = as_bf16x8(r.x[u][1]);
-      // The three products of each pair, four independent accumulators
+      // The three products of each pair, RB independent accumulators
       // between two that update the same one.
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, wh[i], acc[i], 0, 0, 0);
+      for (int i = 0; i < RB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, wh[i], acc[i], 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xl, wh[i], acc[i], 0, 0, 0);
+      for (int i = 0; i < RB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xl, wh[i], acc[i], 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, wl[i], acc[i], 0, 0, 0);
+      for (int i = 0; i < RB; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, wl[i], acc[i], 0, 0, 0);
     }
   };
-  // Weights run three blocks ahead in three register sets, tokens two
-  // ahead in two. Block kb: the next block's weights (loaded two blocks
-  // ago) go to the other LDS buffer and block kb + 3's are requested into
-  // their set; this block's products run from this buffer and this block's
-  // token fragments; then block kb + 2's tokens are requested into theirs.
-  // Every load is issued whatever kb (past the last block it reloads the
-  // last), so the waits count exactly the loads they need.
-  WeightLoad2 wa = load_w(kb0);
-  TokenLoad xa = load_x(kb0);
-  WeightLoad2 wb = load_w(min(kb0 + 1, kb1 - 1));
-  TokenLoad xb = load_x(min(kb0 + 1, kb1 - 1));
-  WeightLoad2 wc = load_w(min(kb0 + 2, kb1 - 1));
-  put(stage[0], wa);
+  // Weights run kW blocks ahead, tokens kX. Block kb: the next block's weights
+  // go to the other LDS buffer and block kb + 1 + kW's are requested into their
+  // set; this block's products run from this buffer and this block's token
+  // fragments; then block kb + kX's tokens are requested into theirs. Loads
+  // return in order, so a wait for tokens is also one for the weights asked
+  // for before them. Every load is issued whatever kb (past the last block it
+  // reloads the last), so the waits count exactly the loads they need.
+  WeightLoad2 ws[kW];
+  TokenLoad xs[kX];
+  // In the order the loop asks for them: block i's tokens after block
+  // i + kW + 1 - kX's weights.
+#pragma unroll
+  for (int d = 0; d <= kW; ++d) {
+    if (d == kW) put(stage[0], ws[0]);
+    ws[d % kW] = load_w(min(kb0 + d, kb1 - 1));
+    const int i = d - (kW + 1 - kX);
+    if (i >= 0) xs[i] = load_x(min(kb0 + i, kb1 - 1));
+    __builtin_amdgcn_sched_barrier(0);
+  }
   __syncthreads();
-  auto block_step = [&](int kb, const uint4 (&cur)[2][4][2][64], uint4 (&next)[2][4][2][64],
-                        WeightLoad2& w_free, const WeightLoad2& w_next, TokenLoad& x_cur) {
-    put(next, w_next);  // read before the previous barrier
-    w_free = load_w(min(kb + 3, kb1 - 1));
-    compute(cur, x_cur);
-    x_cur = load_x(min(kb + 2, kb1 - 1));
+  static_assert(kW % kX == 0 && kW % 2 == 0, "a turn of kW blocks ends where it began");
+  auto block_step = [&](int kb, int d) {
+    put(stage[(d + 1) & 1], ws[(d + 1) % kW]);
+    ws[(d + 1) % kW] = load_w(min(kb + 1 + kW, kb1 - 1));
+    if (active) compute(stage[d & 1], xs[d % kX]);
+    xs[d % kX] = load_x(min(kb + kX, kb1 - 1));
     __syncthreads();
   };
-  // LDS buffers and token sets alternate every block, weight sets every
-  // third: six blocks a turn.
-  for (int kb = kb0; kb < kb1; kb += 6) {
-    block_step(kb, stage[0], stage[1], wa, wb, xa);
-    if (kb + 1 >= kb1) break;
-    block_step(kb + 1, stage[1], stage[0], wb, wc, xb);
-    if (kb + 2 >= kb1) break;
-    block_step(kb + 2, stage[0], stage[1], wc, wa, xa);
-    if (kb + 3 >= kb1) break;
-    block_step(kb + 3, stage[1], stage[0], wa, wb, xb);
-    if (kb + 4 >= kb1) break;
-    block_step(kb + 4, stage[0], stage[1], wb, wc, xa);
-    if (kb + 5 >= kb1) break;
-    block_step(kb + 5, stage[1], stage[0], wc, wa, xb);
+  // Whole turns, then the rest apart: an exit inside the turn would make every
+  // turn's first waits the exit's, for loads just asked for.
+  int kb = kb0;
+  for (; kb + kW <= kb1; kb += kW) {
+#pragma unroll
+    for (int d = 0; d < kW; ++d) block_step(kb + d, d);
+  }
+#pragma unroll
+  for (int d = 0; d < kW - 1; ++d) {
+    if (kb + d < kb1) block_step(kb + d, d);
   }
 
   // Lane l's register e of a 32 x 32 block: token (e / 4) 8 + (l / 32) 4 +
@@ -389,12 +402,12 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(const DevSte
     const uint32_t first = g.edits ? g.edits[2 * g.layer] : 0u;
     const uint32_t count = g.edits ? g.edits[2 * g.layer + 1] : 0u;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int n = rt * (kTileRows / 2) + i * 32 + row_in;
+    for (int i = 0; i < RB / 2; ++i) {
+      const int n = rt * (kTileRows / 2) + tile_block(i) * 32 + row_in;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int t = n0 + wave * 32 + (e >> 2) * 8 + tok_in + (e & 3);
-        float v = gelu_fast(acc[i][e]) * acc[i + 2][e];
+        float v = gelu_fast(acc[i][e]) * acc[i + RB / 2][e];
         if (count) v = pin_one(g.edits, first, count, n, step->position + (uint32_t)t, v);
         if (t >= tokens || n >= g.rows) continue;
         if (g.y) g.y[(size_t)t * g.ldy + n] = v;
@@ -408,8 +421,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_bf16_kernel(const DevSte
   }
   float* y = g.y + (size_t)z * g.part_stride;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int o = rt * kTileRows + i * 32 + row_in;
+  for (int i = 0; i < RB; ++i) {
+    const int o = rt * kTileRows + tile_block(i) * 32 + row_in;
     if (o >= g.rows) continue;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -451,6 +464,12 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const DevStep* __restric
     y[at] = v;
   }
 }
+
+// A step of one token tile takes half tiles of rows: gate and up's 108 tiles
+// leave most CUs idle, and what binds a workgroup then is the weights it has
+// in flight. 150 tokens of Gemma-3-1B 3.39 -> 2.87 ms, 256 3.60 -> 3.30; two
+// token tiles (300 tokens) 3.73 and 3.80, 512 4.28 and 4.38.
+bool half_tiles(int max_tokens) { return max_tokens <= kTileTokens; }
 
 int row_tiles_of(int rows, bool gated) {
   return gated ? (rows + kTileRows / 2 - 1) / (kTileRows / 2) : (rows + kTileRows - 1) / kTileRows;
@@ -498,7 +517,8 @@ int bf16_splits_for(int rows, int cols, int max_tokens, bool gated) {
   // As many workgroups as the 256 CUs hold (one each), at least two K
   // blocks a split, and no split left empty.
   if (gated) return 1;
-  const int tiles = row_tiles_of(rows, false) * ((max_tokens + kTileTokens - 1) / kTileTokens);
+  const int tiles = row_tiles_of(rows, false) * (half_tiles(max_tokens) ? 2 : 1) *
+                    ((max_tokens + kTileTokens - 1) / kTileTokens);
   const int blocks = cols / 32;
   int splits = std::min({kMaxBf16Splits, std::max(1, 256 / tiles), std::max(1, blocks / 2)});
   const int per = (blocks + splits - 1) / splits;
@@ -518,10 +538,14 @@ hipError_t launch_gemm_bf16(hipStream_t s, const DevStep* step, Bf16Gemm g, int 
   g.k_blocks = (blocks + splits - 1) / splits;
   g.token_tiles = (max_tokens + kTileTokens - 1) / kTileTokens;
   const int tiles = row_tiles_of(g.rows, g.gated) * splits * g.token_tiles;
+  const bool half = half_tiles(max_tokens);
+  auto launch = [&](auto kernel, int n) {
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(kGemmThreads), 0, s, step, g);
+  };
   if (g.gated) {
-    hipLaunchKernelGGL(gemm_bf16_kernel<true>, dim3(tiles), dim3(kGemmThreads), 0, s, step, g);
+    half ? launch(gemm_bf16_kernel<true, 2>, 2 * tiles) : launch(gemm_bf16_kernel<true, 4>, tiles);
   } else {
-    hipLaunchKernelGGL(gemm_bf16_kernel<false>, dim3(tiles), dim3(kGemmThreads), 0, s, step, g);
+    half ? launch(gemm_bf16_kernel<false, 2>, 2 * tiles) : launch(gemm_bf16_kernel<false, 4>, tiles);
   }
   return hipGetLastError();
 }

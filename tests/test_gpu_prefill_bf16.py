@@ -77,6 +77,14 @@ def test_gemm_bf16_within_bound(device, rows, cols, tokens, splits, fmt):
     assert float(np.median(err / (np.abs(x.astype(np.float64)) @ np.abs(w64).T))) < 2.0 ** -16
 
 
+# Steps of one token tile (at most 256 tokens) take half tiles of rows; the K
+# loop runs in turns of four blocks.
+@pytest.mark.parametrize("rows,tokens", [(60, 256), (60, 257), (132, 33)])
+@pytest.mark.parametrize("cols,splits", [(32, 1), (96, 1), (128, 1), (160, 1), (288, 2)])
+def test_gemm_bf16_at_the_tiles_edges(device, rows, tokens, cols, splits):
+    test_gemm_bf16_within_bound(device, rows, cols, tokens, splits, fz.Q4_0)
+
+
 def test_gated_bf16_within_bound_with_pins(device):
     rows, cols, tokens, position = 6912, 1152, 200, 40
     rng = np.random.default_rng(7)
