@@ -1249,6 +1249,12 @@ bool pass_tiles(const QMatrix& w, int max_tokens, int x_stride) {
   return (many || max_tokens <= Mfma<4>::kDim) && groups >= kRanges;
 }
 
+bool pass_pairs(const QMatrix& w, int max_tokens) {
+  const int pairs = (w.rows + 2 * Mfma<4>::kDim - 1) / (2 * Mfma<4>::kDim);
+  return (w.cols >> 5) <= 2 * kRanges &&
+         pairs * ((max_tokens + Mfma<4>::kDim - 1) / Mfma<4>::kDim) >= 384;
+}
+
 }  // namespace
 
 hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
@@ -1271,9 +1277,14 @@ hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
   if (pass_tiles(w, max_tokens, x_stride)) {
     switch (w.format) {
       case kQ4_0:
-        // Thousands of tiles (a vocabulary's head) go a pair to a wave: half
-        // the input traffic, two chains in flight.
-        if (w.rows >= 2048 * Mfma<4>::kDim)
+        // Tiles go a pair to a wave (half the input traffic, two chains in
+        // flight) where the pairs' workgroups keep the chip busy: a vocabulary's
+        // head, and K of at most 64 groups from 384 of them on. Q/K/V took, a
+        // tile then a pair, 7.7 and 7.9 us at 64 rows (192 workgroups), 11.4 and
+        // 11.1 at 128 (384), 35 and 28 at 512; O 9.0 and 9.3 at 128 (288), 13.5
+        // and 13.2 at 256 (576). Longer K keeps a workgroup a CU: down was no
+        // faster in pairs (116 and 114 us at 512 rows, 65 and 69 at 256).
+        if (w.rows >= 2048 * Mfma<4>::kDim || pass_pairs(w, max_tokens))
           return launch_pass_tiles<kPairKind, kQ4_0>(s, step, w, w, x, x_stride, y, y_stride,
                                                      max_tokens, nullptr, 0);
         return launch_pass_tiles<kPlainKind, kQ4_0>(s, step, w, w, x, x_stride, y, y_stride,

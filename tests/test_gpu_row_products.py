@@ -31,6 +31,8 @@ def _check_rows(got, want_row, tokens):
     (2, 8191, 1152, 17), (3, 1152, 6912, 49), (8, 1152, 6912, 130), (3, 40, 1152, 300),
     (2, 1152, 6912, 497), (2, 1536, 1152, 512), (2, 1152, 1024, 401), (8, 36, 6912, 512),
     (3, 36, 6912, 511), (2, 40, 992, 77), (2, 40, 16416, 17),
+    (2, 1536, 1152, 113), (2, 1500, 1152, 300), (2, 1137, 1024, 176), (2, 600, 2048, 512),
+    (2, 600, 2080, 512),
     (2, 1152, 1056, 19)])
 def test_row_products_bit_exact(device, fmt, rows, cols, tokens):
     rng = np.random.default_rng(rows + cols + tokens)
