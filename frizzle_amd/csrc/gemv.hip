@@ -17,9 +17,12 @@
 #include "edit_common.h"
 #include "kernels.h"
 #include "numerics.h"
+#include "product_rules.h"
 
 namespace frz {
 namespace {
+
+static_assert(rules::kRanges == kRanges, "the rules count the kernels' ranges");
 
 __device__ __forceinline__ float half_to_float(uint16_t h) {
   return (float)__builtin_bit_cast(_Float16, h);
@@ -1235,18 +1238,14 @@ hipError_t launch_wide(hipStream_t s, const DevStep* step, QMatrix gate, QMatrix
   return hipGetLastError();
 }
 
-// A step over K of 32 groups or more takes a pass a wave, whose workgroups are
-// small enough to fill the chip at every row count and to even out its last
-// round. gemm_ranges, a wave a tile, took for Q/K/V, O and down 25, 18 and 90
-// us at 288 rows and 38, 24 and 121 at 512; a pass a wave 23, 16 and 75, and
-// 34, 23 and 112. A matrix of thousands of tiles (the vocabulary's) fills the
-// chip a wave a tile from 17 rows on.
+// Whether a product takes a pass a wave (product_rules.h).
 bool pass_tiles(const QMatrix& w, int max_tokens, int x_stride) {
   const int groups = w.cols >> 5;
   // Past 16 rows, only what gemm_ranges would take as well.
-  const bool many = w.rows < 512 * Mfma<4>::kDim && groups <= kWideGroups &&
-                    4ull * (uint64_t)x_stride * (uint64_t)max_tokens < kPastEnd;
-  return (many || max_tokens <= Mfma<4>::kDim) && groups >= kRanges;
+  if (max_tokens > Mfma<4>::kDim &&
+      (groups > kWideGroups || 4ull * (uint64_t)x_stride * (uint64_t)max_tokens >= kPastEnd))
+    return false;
+  return rules::takes_pass(w.format == kQ4_0, w.rows, groups, max_tokens);
 }
 
 bool pass_pairs(const QMatrix& w, int max_tokens) {
@@ -1268,12 +1267,7 @@ hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
     in.x = x + (size_t)(last_token ? max_tokens - 1 : 0) * x_stride;
     return launch_gemv_decode(s, step, w, in, 0, y);
   }
-  // Tiles of 32 x 32 (two ranges in flight) when they are enough to cover
-  // most of the chip's 1,024 SIMDs; else 16 x 16 tiles (four ranges), four
-  // times as many.
-  // 32 x 32 tiles waste half their columns on 16 tokens or fewer.
-  const bool wide = (size_t)w.rows * (size_t)max_tokens >= (size_t)768 * 1024 &&
-                    max_tokens > Mfma<4>::kDim;
+  const bool wide = rules::wide_chain(w.rows, max_tokens);
   if (pass_tiles(w, max_tokens, x_stride)) {
     switch (w.format) {
       case kQ4_0:
@@ -1358,7 +1352,11 @@ hipError_t launch_gated(hipStream_t s, const DevStep* step, QMatrix gate,
     in.x = x;
     return launch_gated_decode(s, step, gate, up, in, 0, act, edits, layer);
   }
-  if (pass_tiles(gate, max_tokens, gate.cols) && max_tokens <= kGatedPassRows) {
+  const int groups = gate.cols >> 5;
+  const bool many = gate.rows < 512 * Mfma<4>::kDim && groups <= kWideGroups &&
+                    4ull * (uint64_t)gate.cols * (uint64_t)max_tokens < kPastEnd;
+  if ((many || max_tokens <= Mfma<4>::kDim) && groups >= kRanges &&
+      max_tokens <= kGatedPassRows) {
     return launch_pass_tiles<kGatedKind, kQ4_0>(s, step, gate, up, x, gate.cols, act, gate.rows,
                                           max_tokens, edits, layer, edit_stride);
   }

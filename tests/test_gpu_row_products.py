@@ -33,7 +33,9 @@ def _check_rows(got, want_row, tokens):
     (3, 36, 6912, 511), (2, 40, 992, 77), (2, 40, 16416, 17),
     (2, 1536, 1152, 113), (2, 1500, 1152, 300), (2, 1137, 1024, 176), (2, 600, 2048, 512),
     (2, 600, 2080, 512),
-    (2, 1152, 1056, 19)])
+    (2, 1152, 1056, 19),
+    # Where a wave a tile is sooner: 32 x 32 tiles, and 16 x 16 ones.
+    (2, 4096, 1152, 512), (3, 1600, 2080, 500), (8, 1024, 4096, 512)])
 def test_row_products_bit_exact(device, fmt, rows, cols, tokens):
     rng = np.random.default_rng(rows + cols + tokens)
     w = format_blocks(rng, fmt, rows, cols)
