@@ -49,7 +49,8 @@ __device__ __forceinline__ float half_to_float(uint16_t h) {
 // token's inputs for that group. So every lane does distinct work and a pass
 // keeps NB chains in flight. The inputs of a step (NB groups x D tokens = 64
 // lines of 32 floats) are loaded whole-line into LDS and read back one line
-// per lane.
+// per lane. A gated wave holds the gate and up tiles of the same neurons,
+// sharing the inputs.
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v32f __attribute__((ext_vector_type(32)));
@@ -227,11 +228,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* base, ui
 constexpr int kXLine = 9;
 constexpr int kXBuf = 64 * kXLine;
 
-template <int NB>
+template <int NB, bool GATED>
 struct Tile {
   static constexpr int D = Mfma<NB>::kDim;
   static constexpr int kTokenRows = 8 / NB;  // distinct tokens a lane loads
-  __amdgpu_buffer_rsrc_t x, codes, scales;
+  static constexpr int kMats = GATED ? 2 : 1;
+  __amdgpu_buffer_rsrc_t x, codes[kMats], scales[kMats];
   uint32_t x_off[kTokenRows];  // byte offset of float4 lane % 8 of each token it loads
   uint32_t row_group0;         // this lane's row times the row's groups
   float4* x_put;               // its load slots (+ 8 kXLine i)
@@ -242,10 +244,10 @@ struct Tile {
 // Step t's inputs: instruction i is lines 8 i .. 8 i + 7, block
 // i / (8 / NB). A finished block's lines are loaded (from a valid group)
 // and zeroed when staged.
-template <int NB>
-__device__ __forceinline__ void load_inputs(const Tile<NB>& T, const StepInfo<NB>& I,
+template <int NB, bool GATED>
+__device__ __forceinline__ void load_inputs(const Tile<NB, GATED>& T, const StepInfo<NB>& I,
                                             float4 (&G)[8]) {
-  constexpr int kPer = Tile<NB>::kTokenRows;
+  constexpr int kPer = Tile<NB, GATED>::kTokenRows;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const uint32_t g = I.entry(i / kPer) & 0x7FFFu;
@@ -254,10 +256,10 @@ __device__ __forceinline__ void load_inputs(const Tile<NB>& T, const StepInfo<NB
   }
 }
 
-template <int NB>
-__device__ __forceinline__ void stage_inputs(const Tile<NB>& T, const StepInfo<NB>& I,
+template <int NB, bool GATED>
+__device__ __forceinline__ void stage_inputs(const Tile<NB, GATED>& T, const StepInfo<NB>& I,
                                              float4 (&G)[8]) {
-  constexpr int kPer = Tile<NB>::kTokenRows;
+  constexpr int kPer = Tile<NB, GATED>::kTokenRows;
   if (I.flags & kPads) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -286,50 +288,60 @@ struct Weights<false, kQ4_1> {
   uint32_t d[1];  // d, then m in the high half
 };
 
-template <int NB, int F>
-__device__ __forceinline__ void load_weights(const Tile<NB>& T, const StepInfo<NB>& I,
-                                             Weights<false, F>& W) {
+template <int NB, bool GATED, int F>
+__device__ __forceinline__ void load_weights(const Tile<NB, GATED>& T, const StepInfo<NB>& I,
+                                             Weights<GATED, F>& W) {
   // this lane's block's group
   uint32_t g = I.entry(0);
 #pragma unroll
   for (int b = 1; b < NB; ++b) g = T.block == b ? I.entry(b) : g;
   const uint32_t blk = T.row_group0 + (g & 0x7FFFu);
-  const uint32_t code_at = (uint32_t)code_bytes(F) * blk;
-  W.c[0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(T.codes, code_at, 0, 0));
-  if constexpr (F == kQ8_0) {
-    W.c[1] = __builtin_bit_cast(
-        uint4, __builtin_amdgcn_raw_buffer_load_b128(T.codes, code_at + 16, 0, 0));
-  }
-  if constexpr (F == kQ4_1) {
-    W.d[0] = __builtin_amdgcn_raw_buffer_load_b32(T.scales, 4 * blk, 0, 0);
-  } else {
-    W.d[0] = __builtin_amdgcn_raw_buffer_load_b16(T.scales, 2 * blk, 0, 0);
+#pragma unroll
+  for (int m = 0; m < Tile<NB, GATED>::kMats; ++m) {
+    if constexpr (F == kQ8_0) {
+      W.c[0] = __builtin_bit_cast(uint4,
+                                  __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 32 * blk, 0, 0));
+      W.c[1] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 32 * blk + 16, 0, 0));
+      W.d[0] = __builtin_amdgcn_raw_buffer_load_b16(T.scales[m], 2 * blk, 0, 0);
+    } else if constexpr (F == kQ4_1) {
+      W.c[0] = __builtin_bit_cast(uint4,
+                                  __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 16 * blk, 0, 0));
+      W.d[0] = __builtin_amdgcn_raw_buffer_load_b32(T.scales[m], 4 * blk, 0, 0);
+    } else {
+      W.c[m] = __builtin_bit_cast(uint4,
+                                  __builtin_amdgcn_raw_buffer_load_b128(T.codes[m], 16 * blk, 0, 0));
+      W.d[m] = __builtin_amdgcn_raw_buffer_load_b16(T.scales[m], 2 * blk, 0, 0);
+    }
   }
 }
 
-// Products for k = 16 H .. 16 H + 15 of a step: decode the weights, then the
-// 16 products per block.
-template <int NB, int F, int H>
-__device__ __forceinline__ void chain_half(const float4 (&xv)[8], const Weights<false, F>& W,
-                                           typename Mfma<NB>::Acc& acc) {
-  float wk[16];
-  if constexpr (F == kQ8_0) {
-    decode_half_q8_0(W.c[H], W.d[0], wk);
-  } else if constexpr (F == kQ4_1) {
-    decode_half_q4_1<H>(W.c[0], W.d[0], wk);
-  } else {
-    decode_half<H>(W.c[0], W.d[0], wk);
-  }
-  __builtin_amdgcn_sched_barrier(0);
+// Products for k = 16 H .. 16 H + 15 of a step, per matrix: decode the
+// weights, then the 16 products per block.
+template <int NB, bool GATED, int F, int H>
+__device__ __forceinline__ void chain_half(const float4 (&xv)[8], const Weights<GATED, F>& W,
+                                           typename Mfma<NB>::Acc (&acc)[GATED ? 2 : 1]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float4 x4 = xv[4 * H + i];
-    acc = Mfma<NB>::op(wk[4 * i + 0], x4.x, acc);
-    acc = Mfma<NB>::op(wk[4 * i + 1], x4.y, acc);
-    acc = Mfma<NB>::op(wk[4 * i + 2], x4.z, acc);
-    acc = Mfma<NB>::op(wk[4 * i + 3], x4.w, acc);
+  for (int m = 0; m < (GATED ? 2 : 1); ++m) {
+    float wk[16];
+    if constexpr (F == kQ8_0) {
+      decode_half_q8_0(W.c[H], W.d[0], wk);
+    } else if constexpr (F == kQ4_1) {
+      decode_half_q4_1<H>(W.c[0], W.d[0], wk);
+    } else {
+      decode_half<H>(W.c[m], W.d[m], wk);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float4 x4 = xv[4 * H + i];
+      acc[m] = Mfma<NB>::op(wk[4 * i + 0], x4.x, acc[m]);
+      acc[m] = Mfma<NB>::op(wk[4 * i + 1], x4.y, acc[m]);
+      acc[m] = Mfma<NB>::op(wk[4 * i + 2], x4.z, acc[m]);
+      acc[m] = Mfma<NB>::op(wk[4 * i + 3], x4.w, acc[m]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __builtin_amdgcn_sched_barrier(0);
 }
 
 // Two Q4_0 chains on the same inputs (gate and up, or two tiles), quarter Q
@@ -369,11 +381,11 @@ __device__ __forceinline__ void chain_half_two(const float4 (&xv)[8], const Weig
 // chain this step's 32 products per block, half a group at a time so that
 // the decoded weights need few registers. Vector instructions do not run
 // beside the fp32 matrix instructions, so each kind is kept in runs.
-template <int NB, int F>
-__device__ __forceinline__ void chain_step(const Tile<NB>& T, const StepInfo<NB>& I1,
+template <int NB, bool GATED, int F>
+__device__ __forceinline__ void chain_step(const Tile<NB, GATED>& T, const StepInfo<NB>& I1,
                                            const StepInfo<NB>& I2, float4 (&G)[8],
-                                           const Weights<false, F>& W, Weights<false, F>& W_next,
-                                           typename Mfma<NB>::Acc& acc) {
+                                           const Weights<GATED, F>& W, Weights<GATED, F>& W_next,
+                                           typename Mfma<NB>::Acc (&acc)[GATED ? 2 : 1]) {
   float4 xv[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) xv[i] = T.x_get[i];
@@ -383,8 +395,8 @@ __device__ __forceinline__ void chain_step(const Tile<NB>& T, const StepInfo<NB>
   load_weights(T, I1, W_next);
   // The loads stay here, a step ahead of their use.
   __builtin_amdgcn_sched_barrier(0);
-  chain_half<NB, F, 0>(xv, W, acc);
-  chain_half<NB, F, 1>(xv, W, acc);
+  chain_half<NB, GATED, F, 0>(xv, W, acc);
+  chain_half<NB, GATED, F, 1>(xv, W, acc);
   wave_sync();
 }
 
@@ -404,15 +416,18 @@ __device__ __forceinline__ void close_pass(typename Mfma<NB>::Acc& acc,
 
 // Step t, with the schedule of steps t .. t + 2 in hand; starts reading
 // step t + 3's (first used a step later, so its wait costs nothing).
-template <int NB, int F>
-__device__ __forceinline__ void run_step(const Tile<NB>& T, const Schedule<NB>& S, int t,
+template <int NB, bool GATED, int F>
+__device__ __forceinline__ void run_step(const Tile<NB, GATED>& T, const Schedule<NB>& S, int t,
                                          StepInfo<NB> (&I)[4], float4 (&G)[8],
-                                         const Weights<false, F>& W, Weights<false, F>& W_next,
-                                         typename Mfma<NB>::Acc& acc,
-                                         float (&total)[Mfma<NB>::kSlots]) {
+                                         const Weights<GATED, F>& W, Weights<GATED, F>& W_next,
+                                         typename Mfma<NB>::Acc (&acc)[GATED ? 2 : 1],
+                                         float (&total)[GATED ? 2 : 1][Mfma<NB>::kSlots]) {
   I[3] = step_info(S, t + 3);
-  chain_step<NB, F>(T, I[1], I[2], G, W, W_next, acc);
-  if (I[0].flags & kCloses) close_pass<NB>(acc, total);
+  chain_step<NB, GATED, F>(T, I[1], I[2], G, W, W_next, acc);
+  if (I[0].flags & kCloses) {
+#pragma unroll
+    for (int m = 0; m < (GATED ? 2 : 1); ++m) close_pass<NB>(acc[m], total[m]);
+  }
   I[0] = I[1];
   I[1] = I[2];
   I[2] = I[3];
@@ -420,13 +435,16 @@ __device__ __forceinline__ void run_step(const Tile<NB>& T, const Schedule<NB>& 
 
 // Grid: x = D-row tiles, y = groups of kTileWaves x D tokens, a wave's own
 // D tokens. Rows and tokens past the ends are read clamped and not stored.
-template <int NB, int F = kQ4_0>
+template <int NB, bool GATED, int F = kQ4_0>
 __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
-    const DevStep* __restrict__ step, QMatrix w, const float* __restrict__ x, int x_stride,
-    uint32_t x_bytes, float* __restrict__ y, int y_stride, const Schedule<NB> S) {
+    const DevStep* __restrict__ step, QMatrix w, QMatrix up,
+    const float* __restrict__ x, int x_stride, uint32_t x_bytes, float* __restrict__ y,
+    int y_stride, const uint32_t* __restrict__ edits, int layer, uint32_t edit_stride,
+    const Schedule<NB> S) {
   using M = Mfma<NB>;
   constexpr int D = M::kDim;
   constexpr int SL = M::kSlots;
+  constexpr int kMats = GATED ? 2 : 1;
   __shared__ float4 staged[kTileWaves][kXBuf];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int tokens = (int)step->tokens;
@@ -435,7 +453,7 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
   if (token0 >= tokens) return;
   const int groups = w.cols >> 5;
 
-  Tile<NB> T;
+  Tile<NB, GATED> T;
   T.block = lane / D;
   const int row = min((int)blockIdx.x * D + lane % D, w.rows - 1);
   // The tile's member (a fused product over members placed apart): members
@@ -448,11 +466,15 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
                                             : w.rows;
   const uint32_t blocks = (uint32_t)member_rows * (uint32_t)groups;
   T.row_group0 = (uint32_t)(row - ((int)blockIdx.x * D - mr.row)) * (uint32_t)groups;
-  T.codes = buffer_of(mr.codes, (uint32_t)code_bytes(F) * blocks);
-  T.scales = buffer_of(mr.scales, 2u * (uint32_t)scale_halves(F) * blocks);
+  T.codes[0] = buffer_of(mr.codes, (uint32_t)code_bytes(F) * blocks);
+  T.scales[0] = buffer_of(mr.scales, 2u * (uint32_t)scale_halves(F) * blocks);
+  if (GATED) {
+    T.codes[kMats - 1] = buffer_of(up.codes, 16 * blocks);
+    T.scales[kMats - 1] = buffer_of(up.scales, 2 * blocks);
+  }
   T.x = buffer_of(x, x_bytes);
 #pragma unroll
-  for (int i = 0; i < Tile<NB>::kTokenRows; ++i) {
+  for (int i = 0; i < Tile<NB, GATED>::kTokenRows; ++i) {
     // line 8 i + lane / 8 is token (8 i + lane / 8) % D
     const int tok = min(token0 + (8 * i + (lane >> 3)) % D, tokens - 1);
     T.x_off[i] = 4u * ((uint32_t)tok * (uint32_t)x_stride + 4u * (uint32_t)(lane & 7));
@@ -460,12 +482,15 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
   T.x_put = staged[wave] + (lane >> 3) * kXLine + (lane & 7);
   T.x_get = staged[wave] + lane * kXLine;
 
-  typename M::Acc acc;
-  float total[SL];
+  typename M::Acc acc[kMats];
+  float total[kMats][SL];
 #pragma unroll
-  for (int i = 0; i < NB * SL; ++i) acc[i] = 0.0f;
+  for (int m = 0; m < kMats; ++m) {
 #pragma unroll
-  for (int o = 0; o < SL; ++o) total[o] = 0.0f;
+    for (int i = 0; i < NB * SL; ++i) acc[m][i] = 0.0f;
+#pragma unroll
+    for (int o = 0; o < SL; ++o) total[m][o] = 0.0f;
+  }
 
   // Step 0 staged; step 1's inputs and step 0's weights in registers.
   StepInfo<NB> I[4];
@@ -476,23 +501,33 @@ __global__ __launch_bounds__(kTileWaves * 64) void gemm_ranges(
   load_inputs(T, I[0], G);
   stage_inputs(T, I[0], G);
   load_inputs(T, I[1], G);
-  Weights<false, F> W0, W1;
+  Weights<GATED, F> W0, W1;
   load_weights(T, I[0], W0);
   wave_sync();
   for (int t = 0; t < S.steps; t += 2) {
-    run_step<NB, F>(T, S, t, I, G, W0, W1, acc, total);
+    run_step<NB, GATED, F>(T, S, t, I, G, W0, W1, acc, total);
     if (t + 1 >= S.steps) break;
-    run_step<NB, F>(T, S, t + 1, I, G, W1, W0, acc, total);
+    run_step<NB, GATED, F>(T, S, t + 1, I, G, W1, W0, acc, total);
   }
 
   const int tok = token0 + lane % D;
   if (tok >= tokens) return;
   float* yrow = y + (size_t)tok * y_stride;
   const int row0 = blockIdx.x * D;
+  // A variants step: every row at the step's position, under its own table.
+  const uint32_t position = step->position + (step->variants ? 0u : (uint32_t)tok);
+  if (edits && step->variants) edits += (size_t)tok * edit_stride;
 #pragma unroll
   for (int o = 0; o < SL; ++o) {
     const int n = row0 + M::slot_row(lane, o);
-    if (n < w.rows) yrow[n] = total[o];
+    if (n >= w.rows) continue;
+    if (!GATED) {
+      yrow[n] = total[0][o];
+    } else {
+      float v = gelu_tanh(total[0][o]) * total[kMats - 1][o];
+      if (edits) v = apply_edits(edits, layer, (uint32_t)n, position, v);
+      yrow[n] = v;
+    }
   }
 }
 
@@ -634,12 +669,12 @@ __device__ __forceinline__ void load_pass_weights(const PassLane<GATED, F>& L, i
 template <bool GATED, int F>
 __device__ __forceinline__ void pass_products(const float4 (&xv)[8], const Weights<GATED, F>& W,
                                               typename Mfma<4>::Acc (&acc)[GATED ? 2 : 1]) {
-  if constexpr (GATED) {
+  if constexpr (GATED && F == kQ4_0) {
     chain_half_two<0>(xv, W, acc);
     chain_half_two<1>(xv, W, acc);
   } else {
-    chain_half<4, F, 0>(xv, W, acc[0]);
-    chain_half<4, F, 1>(xv, W, acc[0]);
+    chain_half<4, GATED, F, 0>(xv, W, acc);
+    chain_half<4, GATED, F, 1>(xv, W, acc);
   }
 }
 
@@ -1186,9 +1221,10 @@ hipError_t launch_pass_tiles(hipStream_t s, const DevStep* step, QMatrix w, QMat
   return hipGetLastError();
 }
 
-template <int NB, int F = kQ4_0>
-hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, const float* x,
-                         int x_stride, float* y, int y_stride, int max_tokens) {
+template <int NB, bool GATED, int F = kQ4_0>
+hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, QMatrix up, const float* x,
+                         int x_stride, float* y, int y_stride, int max_tokens,
+                         const uint32_t* edits = nullptr, int layer = 0, uint32_t edit_stride = 0) {
   constexpr int D = Mfma<NB>::kDim;
   const int groups = w.cols >> 5;
   const uint64_t x_bytes = 4ull * (uint64_t)x_stride * (uint64_t)max_tokens;
@@ -1200,15 +1236,10 @@ hipError_t launch_ranges(hipStream_t s, const DevStep* step, QMatrix w, const fl
   }
   const int token_span = kTileWaves * D;
   const dim3 grid((w.rows + D - 1) / D, (max_tokens + token_span - 1) / token_span);
-  hipLaunchKernelGGL((gemm_ranges<NB, F>), grid, dim3(kTileWaves * 64), 0, s, step, w, x, x_stride,
-                     (uint32_t)x_bytes, y, y_stride, S);
+  hipLaunchKernelGGL((gemm_ranges<NB, GATED, F>), grid, dim3(kTileWaves * 64), 0, s, step, w, up, x,
+                     x_stride, (uint32_t)x_bytes, y, y_stride, edits, layer, edit_stride, S);
   return hipGetLastError();
 }
-
-// The gated product a pass a wave took 92 us at 192 rows and 120 at 256
-// (6,912 neurons, K = 1,152), its wide tiles 97 and 104: they fill their
-// 128-token spans a step at a time.
-constexpr int kGatedPassRows = 208;
 
 hipError_t launch_wide(hipStream_t s, const DevStep* step, QMatrix gate, QMatrix up,
                        const float* x, float* act, int max_tokens, const uint32_t* edits,
@@ -1225,12 +1256,7 @@ hipError_t launch_wide(hipStream_t s, const DevStep* step, QMatrix gate, QMatrix
                        dim3(kWideWaves * 64), 0, s, step, gate, up, x, (uint32_t)x_bytes, act,
                        edits, layer, edit_stride);
   };
-  // Tiles of 32 neurons do a little better (half the LDS reads a product)
-  // while all their workgroups fit on the 256 CUs at once, three each; past
-  // that the last round is nearly empty, and tiles of 16, four workgroups a
-  // CU, even it out: 198 and 190 us at 512 rows of 6,912 neurons, 143 and 151
-  // at 384, 104 and 113 at 256.
-  if (((gate.rows + 31) / 32) * spans <= 3 * 256) {
+  if (rules::wide_dim(gate.rows, max_tokens) == 32) {
     launch(wide_gated_kernel<2>, 32);
   } else {
     launch(wide_gated_kernel<4>, 16);
@@ -1296,16 +1322,16 @@ hipError_t launch_gemv(hipStream_t s, const DevStep* step, QMatrix w,
   switch (w.format) {
     case kQ4_0:
       if (wide)
-        return launch_ranges<2>(s, step, w, x, x_stride, y, y_stride, max_tokens);
-      return launch_ranges<4>(s, step, w, x, x_stride, y, y_stride, max_tokens);
+        return launch_ranges<2, false>(s, step, w, w, x, x_stride, y, y_stride, max_tokens);
+      return launch_ranges<4, false>(s, step, w, w, x, x_stride, y, y_stride, max_tokens);
     case kQ4_1:
       if (wide)
-        return launch_ranges<2, kQ4_1>(s, step, w, x, x_stride, y, y_stride, max_tokens);
-      return launch_ranges<4, kQ4_1>(s, step, w, x, x_stride, y, y_stride, max_tokens);
+        return launch_ranges<2, false, kQ4_1>(s, step, w, w, x, x_stride, y, y_stride, max_tokens);
+      return launch_ranges<4, false, kQ4_1>(s, step, w, w, x, x_stride, y, y_stride, max_tokens);
     case kQ8_0:
       if (wide)
-        return launch_ranges<2, kQ8_0>(s, step, w, x, x_stride, y, y_stride, max_tokens);
-      return launch_ranges<4, kQ8_0>(s, step, w, x, x_stride, y, y_stride, max_tokens);
+        return launch_ranges<2, false, kQ8_0>(s, step, w, w, x, x_stride, y, y_stride, max_tokens);
+      return launch_ranges<4, false, kQ8_0>(s, step, w, w, x, x_stride, y, y_stride, max_tokens);
     default:
       return hipErrorInvalidValue;
   }
@@ -1353,14 +1379,22 @@ hipError_t launch_gated(hipStream_t s, const DevStep* step, QMatrix gate,
     return launch_gated_decode(s, step, gate, up, in, 0, act, edits, layer);
   }
   const int groups = gate.cols >> 5;
-  const bool many = gate.rows < 512 * Mfma<4>::kDim && groups <= kWideGroups &&
-                    4ull * (uint64_t)gate.cols * (uint64_t)max_tokens < kPastEnd;
-  if ((many || max_tokens <= Mfma<4>::kDim) && groups >= kRanges &&
-      max_tokens <= kGatedPassRows) {
-    return launch_pass_tiles<kGatedKind, kQ4_0>(s, step, gate, up, x, gate.cols, act, gate.rows,
-                                          max_tokens, edits, layer, edit_stride);
+  rules::Gated form = rules::gated_form(gate.rows, groups, max_tokens);
+  // Past 16 rows, only what the other forms would take as well.
+  if (form == rules::Gated::kPass && max_tokens > Mfma<4>::kDim &&
+      (groups > kWideGroups || 4ull * (uint64_t)gate.cols * (uint64_t)max_tokens >= kPastEnd ||
+       16ull * (uint64_t)gate.rows * (uint64_t)groups >= kPastEnd))
+    form = rules::Gated::kWide;
+  switch (form) {
+    case rules::Gated::kPass:
+      return launch_pass_tiles<kGatedKind, kQ4_0>(s, step, gate, up, x, gate.cols, act, gate.rows,
+                                                  max_tokens, edits, layer, edit_stride);
+    case rules::Gated::kChain:
+      return launch_ranges<2, true>(s, step, gate, up, x, gate.cols, act, gate.rows, max_tokens,
+                                    edits, layer, edit_stride);
+    default:
+      return launch_wide(s, step, gate, up, x, act, max_tokens, edits, layer, edit_stride);
   }
-  return launch_wide(s, step, gate, up, x, act, max_tokens, edits, layer, edit_stride);
 }
 
 }  // namespace frz

@@ -93,5 +93,60 @@ inline bool takes_pass(bool q4_0, int rows, int groups, int tokens) {
   return rows < 8192 && pass_us(q4_0, rows, groups, tokens) <= chain_us(rows, groups, tokens);
 }
 
+// ---- gated products ---------------------------------------------------------
+
+// The wide tiles' neurons (their span: 128 tokens). Tiles of 32 read half the
+// LDS a product of tiles of 16; but a CU takes whole tiles, and where its last
+// would be at most half of one, tiles of 16 leave it half idle for half the
+// time. Of 32 and of 16 took 199 and 193 us at 512 rows of 6,912 neurons (K =
+// 1,152; 3.4 tiles a CU), 149 and 162 at 384 (2.5), 206 and 223 for 8,192
+// neurons at 512 (4).
+inline int wide_dim(int rows, int tokens) {
+  const int tiles = ceil_div(rows, 32) * ceil_div(tokens, 128);
+  return ceil_div(tiles, kCus / 2) < 2 * ceil_div(tiles, kCus) ? 16 : 32;
+}
+
+// Microseconds in the three forms: a pass a wave, the wide tiles, and a wave
+// a tile of two ranges at a time; fits to 2,346 measured products (K 640 to
+// 16,384, 64 to 16,384 neurons, 17 to 512 tokens), within 5 to 6% on average.
+inline double gated_pass_us(int rows, int groups, int tokens) {
+  const double tiles = (double)ceil_div(rows, 16) * ceil_div(tokens, 16) / kSimds;
+  const int steps = pass_steps(groups);
+  return (groups <= kShortGroups ? 7.1 + 1.22 * steps : 5.6 + 1.95 * steps) * tiles;
+}
+
+inline double gated_wide_us(int rows, int groups, int tokens) {
+  const int tiles = ceil_div(rows, 32) * ceil_div(tokens, 128);
+  const double rounds =
+      wide_dim(rows, tokens) == 16 ? 0.5 * ceil_div(tiles, kCus / 2) : ceil_div(tiles, kCus);
+  const double waves = (double)ceil_div(rows, 32) * ceil_div(tokens, 32) / kSimds;
+  return 10.0 + groups * (0.31 + 0.75 * rounds + 0.41 * waves);
+}
+
+inline double gated_chain_us(int rows, int groups, int tokens) {
+  const int row_tiles = ceil_div(rows, 32);
+  const double rounds = ceil_div(row_tiles * ceil_div(tokens, 128), kCus);
+  const double waves = (double)row_tiles * ceil_div(tokens, 32) / kSimds;
+  return 12.0 + chain_steps(groups, 2) * (0.57 + 1.41 * rounds + 0.89 * waves);
+}
+
+enum class Gated { kWide, kPass, kChain };
+
+// A pass a wave up to 16 tokens and wherever it is sooner than the better of
+// the others. Of those, the wide tiles gain by chaining one range at a time:
+// none of a pair waits for a longer one (6,912 neurons, K = 1,152 at 512
+// rows: 219 us a wave a tile, 193 wide). Where the ranges are of one length
+// and long nothing is waited for, and a wave a tile, with no barrier, is
+// 3 to 10% sooner (6,912 neurons, K = 4,096: 321 and 333 us at 256 rows).
+inline Gated gated_form(int rows, int groups, int tokens) {
+  if (groups < kRanges) return Gated::kWide;
+  if (tokens <= 16) return Gated::kPass;
+  const bool chain = groups % kRanges == 0 && groups >= 4 * kRanges;
+  const double other =
+      chain ? gated_chain_us(rows, groups, tokens) : gated_wide_us(rows, groups, tokens);
+  if (gated_pass_us(rows, groups, tokens) <= other) return Gated::kPass;
+  return chain ? Gated::kChain : Gated::kWide;
+}
+
 }  // namespace rules
 }  // namespace frz

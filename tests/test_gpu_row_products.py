@@ -47,12 +47,14 @@ def test_row_products_bit_exact(device, fmt, rows, cols, tokens):
     _check_rows(dy.numpy(), lambda t: orc.gemv_format(fmt, w, rows, cols, x[t]), tokens)
 
 
-# Past 208 rows the wide tiles: of 32 neurons while their workgroups fit on the
-# chip at once, else of 16; K of fewer groups than ranges goes there at any rows.
+# A pass a wave, the wide tiles (of 32 neurons or of 16; K of fewer groups than
+# ranges goes there at any rows) and, over long ranges of one length, a wave a
+# tile: each form where product_rules.h takes it.
 @pytest.mark.parametrize("rows,tokens,cols", [
     (6912, 17, 1152), (1000, 48, 1152), (96, 256, 1152), (96, 257, 1152), (100, 512, 1152),
     (95, 208, 1152), (1000, 209, 1152), (6900, 510, 1152), (6900, 385, 1056), (33, 300, 1056),
-    (50, 2, 32), (40, 9, 96), (70, 161, 992), (70, 225, 1024)])
+    (50, 2, 32), (40, 9, 96), (70, 161, 992), (70, 225, 1024),
+    (6900, 380, 1152), (5000, 33, 96), (8200, 33, 1024), (3000, 511, 4096)])
 def test_gated_rows_bit_exact(device, rows, tokens, cols):
     rng = np.random.default_rng(rows + tokens)
     layers, layer, position = 2, 1, 30
