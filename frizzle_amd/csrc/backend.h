@@ -26,7 +26,9 @@ struct frz_device {
   // 1,048,576 logits; longer calls allocate their own): an allocation and
   // its free, which waits for the device, cost more than the selection.
   uint32_t* topk_scratch = nullptr;
-  std::mutex ops;  // held while an op enqueues launches that share a buffer here
+  // Held while a one-kernel op enqueues its launches, so that ops of several
+  // threads run one after another: they share the stream and what is above.
+  std::mutex ops;
 };
 
 namespace frz {

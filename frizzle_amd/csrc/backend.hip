@@ -1,7 +1,8 @@
 // The C ABI's device, buffer and one-kernel entry points (include/
 // frizzle_hip.h). Each op call fills a device-side step record on the
-// device's stream and launches one kernel family there; ops wait for their
-// work so their host arguments need not outlive the call.
+// device's stream and launches one kernel family there, whole before another
+// thread's op; ops wait for their work so their host arguments need not
+// outlive the call.
 
 #include <algorithm>
 #include <cmath>
@@ -132,6 +133,22 @@ int device_finish(frz_device* dev, hipError_t launched, const char* what) {
   if (launched != hipSuccess) return check_hip(launched, what);
   return check_hip(hipStreamSynchronize(dev->stream), what);
 }
+
+namespace {
+// One op: its step record, then what `launch` enqueues, as one piece - the
+// record is the device's one, so another thread's op must not come between
+// them - and the wait for it, with the lock given back.
+template <typename Launch>
+int run_op(frz_device* dev, const DevStep& s, const char* what, Launch launch) {
+  hipError_t e;
+  {
+    std::lock_guard<std::mutex> lock(dev->ops);
+    if (int rc = device_put_step(dev, s)) return rc;
+    e = launch();
+  }
+  return device_finish(dev, e, what);
+}
+}  // namespace
 
 int attention_max_chunks(int window, int slots) {
   const int by_window = (window + kChunkKeys - 1) / kChunkKeys + 1;
@@ -313,11 +330,10 @@ int frz_op_gemv_format(frz_device* dev, int format, const void* codes, const voi
   if (format != kQ4_0 && format != kQ4_1 && format != kQ8_0) {
     return fail(FRZ_ERR_ARGUMENT, "frz_op_gemv: format " + std::to_string(format));
   }
-  if (int rc = device_put_step(dev, host_step(0, tokens))) return rc;
-  return device_finish(dev,
-                       launch_gemv(dev->stream, dev->step, q4(codes, scales, rows, cols, format),
-                                   x, x_stride, y, y_stride, (int)tokens, last_token != 0),
-                       "frz_op_gemv");
+  return run_op(dev, host_step(0, tokens), "frz_op_gemv", [&] {
+    return launch_gemv(dev->stream, dev->step, q4(codes, scales, rows, cols, format), x, x_stride,
+                       y, y_stride, (int)tokens, last_token != 0);
+  });
 }
 
 int frz_op_gated(frz_device* dev, const void* gate_codes, const void* gate_scales,
@@ -327,12 +343,10 @@ int frz_op_gated(frz_device* dev, const void* gate_codes, const void* gate_scale
   if (!shape_ok(rows, cols) || tokens == 0 || tokens > (uint32_t)kPrefillBlock) {
     return fail(FRZ_ERR_ARGUMENT, "frz_op_gated: bad shape or tokens");
   }
-  if (int rc = device_put_step(dev, host_step(position, tokens))) return rc;
-  return device_finish(
-      dev,
-      launch_gated(dev->stream, dev->step, q4(gate_codes, gate_scales, rows, cols),
-                   q4(up_codes, up_scales, rows, cols), x, act, (int)tokens, edits_dev, layer),
-      "frz_op_gated");
+  return run_op(dev, host_step(position, tokens), "frz_op_gated", [&] {
+    return launch_gated(dev->stream, dev->step, q4(gate_codes, gate_scales, rows, cols),
+                        q4(up_codes, up_scales, rows, cols), x, act, (int)tokens, edits_dev, layer);
+  });
 }
 
 // The fast prefill mode's products through the ABI: the weights unpacked
@@ -350,7 +364,6 @@ int frz_op_gemm_bf16(frz_device* dev, int format, const void* codes, const void*
   if (!bf16_gemm_shape_ok(w, cols, y_stride)) {
     return fail(FRZ_ERR_ARGUMENT, "frz_op_gemm_bf16: format or shape");
   }
-  if (int rc = device_put_step(dev, host_step(0, tokens))) return rc;
   if (splits == 0) splits = bf16_splits_for(rows, cols, (int)tokens, false);
   uint16_t *hi = nullptr, *lo = nullptr;
   float* parts = nullptr;
@@ -361,10 +374,8 @@ int frz_op_gemm_bf16(frz_device* dev, int format, const void* codes, const void*
   if (e == hipSuccess) e = hipMalloc(&lo, plane * 2);
   if (e == hipSuccess) e = hipMalloc(&parts, stride * splits * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&planes, bf16_planes_bytes(rows, cols, false));
-  if (e == hipSuccess) e = launch_unpack_planes(dev->stream, w, nullptr, planes);
-  if (e == hipSuccess)
-    e = launch_split_rows(dev->stream, dev->step, x, x_stride, cols, hi, lo, (int)tokens);
-  if (e == hipSuccess) {
+  int rc = check_hip(e, "frz_op_gemm_bf16");
+  if (rc == FRZ_OK) {
     Bf16Gemm g;
     g.w = planes;
     g.rows = rows;
@@ -375,17 +386,22 @@ int frz_op_gemm_bf16(frz_device* dev, int format, const void* codes, const void*
     g.y = parts;
     g.ldy = y_stride;
     g.part_stride = stride;
-    e = launch_gemm_bf16(dev->stream, dev->step, g, (int)tokens, splits);
+    rc = run_op(dev, host_step(0, tokens), "frz_op_gemm_bf16", [&] {
+      hipError_t r = launch_unpack_planes(dev->stream, w, nullptr, planes);
+      if (r == hipSuccess)
+        r = launch_split_rows(dev->stream, dev->step, x, x_stride, cols, hi, lo, (int)tokens);
+      if (r == hipSuccess) r = launch_gemm_bf16(dev->stream, dev->step, g, (int)tokens, splits);
+      if (r == hipSuccess)
+        r = launch_sum_parts(dev->stream, dev->step, parts, stride, splits, rows, y_stride, y,
+                             (int)tokens);
+      return r;
+    });
   }
-  if (e == hipSuccess)
-    e = launch_sum_parts(dev->stream, dev->step, parts, stride, splits, rows, y_stride, y,
-                         (int)tokens);
-  if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
   if (hi) (void)hipFree(hi);
   if (lo) (void)hipFree(lo);
   if (parts) (void)hipFree(parts);
   if (planes) (void)hipFree(planes);
-  return check_hip(e, "frz_op_gemm_bf16");
+  return rc;
 }
 
 int frz_op_gated_bf16(frz_device* dev, const void* gate_codes, const void* gate_scales,
@@ -395,7 +411,6 @@ int frz_op_gated_bf16(frz_device* dev, const void* gate_codes, const void* gate_
   if (!shape_ok(rows, cols) || rows % 16 || tokens == 0 || tokens > (uint32_t)kPrefillBlock) {
     return fail(FRZ_ERR_ARGUMENT, "frz_op_gated_bf16: bad shape or tokens");
   }
-  if (int rc = device_put_step(dev, host_step(position, tokens))) return rc;
   const QMatrix gate = q4(gate_codes, gate_scales, rows, cols);
   const QMatrix up = q4(up_codes, up_scales, rows, cols);
   uint16_t *hi = nullptr, *lo = nullptr;
@@ -405,10 +420,8 @@ int frz_op_gated_bf16(frz_device* dev, const void* gate_codes, const void* gate_
   hipError_t e = hipMalloc(&hi, (in + out) * 2);
   if (e == hipSuccess) e = hipMalloc(&lo, (in + out) * 2);
   if (e == hipSuccess) e = hipMalloc(&planes, bf16_planes_bytes(rows, cols, true));
-  if (e == hipSuccess) e = launch_unpack_planes(dev->stream, gate, &up, planes);
-  if (e == hipSuccess)
-    e = launch_split_rows(dev->stream, dev->step, x, cols, cols, hi, lo, (int)tokens);
-  if (e == hipSuccess) {
+  int rc = check_hip(e, "frz_op_gated_bf16");
+  if (rc == FRZ_OK) {
     Bf16Gemm g;
     g.w = planes;
     g.rows = rows;
@@ -423,13 +436,18 @@ int frz_op_gated_bf16(frz_device* dev, const void* gate_codes, const void* gate_
     g.y_lo = lo + in;
     g.edits = edits_dev;
     g.layer = layer;
-    e = launch_gemm_bf16(dev->stream, dev->step, g, (int)tokens, 1);
+    rc = run_op(dev, host_step(position, tokens), "frz_op_gated_bf16", [&] {
+      hipError_t r = launch_unpack_planes(dev->stream, gate, &up, planes);
+      if (r == hipSuccess)
+        r = launch_split_rows(dev->stream, dev->step, x, cols, cols, hi, lo, (int)tokens);
+      if (r == hipSuccess) r = launch_gemm_bf16(dev->stream, dev->step, g, (int)tokens, 1);
+      return r;
+    });
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(dev->stream);
   if (hi) (void)hipFree(hi);
   if (lo) (void)hipFree(lo);
   if (planes) (void)hipFree(planes);
-  return check_hip(e, "frz_op_gated_bf16");
+  return rc;
 }
 
 int frz_op_norm(frz_device* dev, const float* gain, const float* post_gain, const float* output,
@@ -438,9 +456,9 @@ int frz_op_norm(frz_device* dev, const float* gain, const float* post_gain, cons
   if (width <= 0 || width % 4 != 0 || tokens == 0 || tokens > (uint32_t)kPrefillBlock) {
     return fail(FRZ_ERR_ARGUMENT, "frz_op_norm: bad width or tokens");
   }
-  if (int rc = device_put_step(dev, host_step(0, tokens))) return rc;
   NormArgs a{gain, post_gain, output, hidden, normed, epsilon, width, last_token != 0};
-  return device_finish(dev, launch_norm(dev->stream, dev->step, a, (int)tokens), "frz_op_norm");
+  return run_op(dev, host_step(0, tokens), "frz_op_norm",
+                [&] { return launch_norm(dev->stream, dev->step, a, (int)tokens); });
 }
 
 int frz_op_rope(frz_device* dev, const float* turns, const float* query_gain,
@@ -451,10 +469,10 @@ int frz_op_rope(frz_device* dev, const float* turns, const float* query_gain,
   if (tokens == 0 || tokens > (uint32_t)kPrefillBlock || slots < (int)tokens) {
     return fail(FRZ_ERR_ARGUMENT, "frz_op_rope: bad tokens or slots");
   }
-  if (int rc = device_put_step(dev, host_step(position, tokens))) return rc;
   RopeArgs a{turns, query_gain, key_gain, query, key, value, q_stride, kv_stride,
              key_cache, value_cache, slots, head_dim, query_heads, kv_heads, epsilon};
-  return device_finish(dev, launch_rope(dev->stream, dev->step, a, (int)tokens), "frz_op_rope");
+  return run_op(dev, host_step(position, tokens), "frz_op_rope",
+                [&] { return launch_rope(dev->stream, dev->step, a, (int)tokens); });
 }
 
 int frz_op_attention(frz_device* dev, const float* query, int q_stride,
@@ -472,15 +490,12 @@ int frz_op_attention(frz_device* dev, const float* query, int q_stride,
   if (int rc = check_hip(hipMalloc(&partials, (part_floats + stat_floats) * sizeof(float)),
                          "hipMalloc(partials)"))
     return rc;
-  int rc = device_put_step(dev, host_step(position, tokens));
-  if (rc == FRZ_OK) {
-    const float scale_log2e = (float)((double)scale * 1.4426950408889634);
-    AttentionArgs a{query,    q_stride, key_cache,  value_cache, out,       partials,
-                    partials + part_floats, slots, window, head_dim, query_heads,
-                    kv_heads, max_chunks, scale_log2e};
-    rc = device_finish(dev, launch_attention(dev->stream, dev->step, a, (int)tokens),
-                       "frz_op_attention");
-  }
+  const float scale_log2e = (float)((double)scale * 1.4426950408889634);
+  AttentionArgs a{query,    q_stride, key_cache,  value_cache, out,       partials,
+                  partials + part_floats, slots, window, head_dim, query_heads,
+                  kv_heads, max_chunks, scale_log2e};
+  const int rc = run_op(dev, host_step(position, tokens), "frz_op_attention",
+                        [&] { return launch_attention(dev->stream, dev->step, a, (int)tokens); });
   (void)hipFree(partials);
   return rc;
 }
@@ -506,21 +521,20 @@ int frz_op_rope_attention(frz_device* dev, const float* qkv, const float* turns,
   if (int rc = check_hip(hipMalloc(&partials, (part_floats + part_floats / 64) * sizeof(float)),
                          "hipMalloc(partials)"))
     return rc;
-  int rc = device_put_step(dev, host_step(position, 1));
-  if (rc == FRZ_OK) {
-    const float scale_log2e = (float)((double)scale * 1.4426950408889634);
-    DecodeAttentionArgs a{qkv,        turns,    query_gain,            key_gain, key_cache,
-                          value_cache, partials, partials + part_floats, slots,   window,
-                          256,        4,        1,                     max_chunks, epsilon,
-                          scale_log2e};
+  const float scale_log2e = (float)((double)scale * 1.4426950408889634);
+  DecodeAttentionArgs a{qkv,        turns,    query_gain,            key_gain, key_cache,
+                        value_cache, partials, partials + part_floats, slots,   window,
+                        256,        4,        1,                     max_chunks, epsilon,
+                        scale_log2e};
+  const int rc = run_op(dev, host_step(position, 1), "frz_op_rope_attention", [&] {
     hipError_t e = launch_attention_decode(dev->stream, dev->step, a);
     if (e == hipSuccess) {
       e = launch_attention_fold(dev->stream, dev->step,
                                 FoldArgs{partials, partials + part_floats, out, window, max_chunks},
                                 1);
     }
-    rc = device_finish(dev, e, "frz_op_rope_attention");
-  }
+    return e;
+  });
   (void)hipFree(partials);
   return rc;
 }
@@ -556,19 +570,20 @@ int frz_op_rope_attention_noalloc(frz_device* dev, const float* qkv, const float
   // launch, so nothing needs clearing between calls.
   float* partials = dev->static_workspace;
   const size_t part_floats = (size_t)max_chunks * 4 * 256;
-  if (int rc = device_put_step(dev, host_step(position, 1))) return rc;
   const float scale_log2e = (float)((double)scale * 1.4426950408889634);
   DecodeAttentionArgs a{qkv,        turns,    query_gain,            key_gain, key_cache,
                         value_cache, partials, partials + part_floats, slots,   window,
                         256,        4,        1,                     max_chunks, epsilon,
                         scale_log2e};
-  hipError_t e = launch_attention_decode(dev->stream, dev->step, a);
-  if (e == hipSuccess) {
-    e = launch_attention_fold(dev->stream, dev->step,
-                              FoldArgs{partials, partials + part_floats, out, window, max_chunks},
-                              1);
-  }
-  return device_finish(dev, e, "frz_op_rope_attention_noalloc");
+  return run_op(dev, host_step(position, 1), "frz_op_rope_attention_noalloc", [&] {
+    hipError_t e = launch_attention_decode(dev->stream, dev->step, a);
+    if (e == hipSuccess) {
+      e = launch_attention_fold(dev->stream, dev->step,
+                                FoldArgs{partials, partials + part_floats, out, window, max_chunks},
+                                1);
+    }
+    return e;
+  });
 }
 
 int frz_op_gather(frz_device* dev, const void* codes, const void* scales, int rows, int cols,
@@ -588,12 +603,15 @@ int frz_op_gather_format(frz_device* dev, int format, const void* codes, const v
   }
   DevStep s = host_step(0, tokens);
   std::memcpy(s.ids, ids, tokens * sizeof(uint32_t));
-  if (int rc = device_copy_step(dev, s)) return rc;
-  return device_finish(
-      dev,
-      launch_gather(dev->stream, dev->step, q4(codes, scales, rows, cols, format), nullptr,
-                    hidden, scale, (int)tokens),
-      "frz_op_gather");
+  hipError_t e;
+  {
+    // As run_op, with the record's ids.
+    std::lock_guard<std::mutex> lock(dev->ops);
+    if (int rc = device_copy_step(dev, s)) return rc;
+    e = launch_gather(dev->stream, dev->step, q4(codes, scales, rows, cols, format), nullptr,
+                      hidden, scale, (int)tokens);
+  }
+  return device_finish(dev, e, "frz_op_gather");
 }
 
 int frz_op_edit(frz_device* dev, const uint32_t* edits_dev, int layer, float* act, int width,
@@ -601,10 +619,9 @@ int frz_op_edit(frz_device* dev, const uint32_t* edits_dev, int layer, float* ac
   if (tokens == 0 || tokens > (uint32_t)kPrefillBlock) {
     return fail(FRZ_ERR_ARGUMENT, "frz_op_edit: bad tokens");
   }
-  if (int rc = device_put_step(dev, host_step(position, tokens))) return rc;
-  return device_finish(
-      dev, launch_edit(dev->stream, dev->step, edits_dev, layer, act, width, (int)tokens),
-      "frz_op_edit");
+  return run_op(dev, host_step(position, tokens), "frz_op_edit", [&] {
+    return launch_edit(dev->stream, dev->step, edits_dev, layer, act, width, (int)tokens);
+  });
 }
 
 int frz_op_topk(frz_device* dev, const float* logits, int count, uint32_t* candidates_dev) {
@@ -636,10 +653,9 @@ int frz_op_draw(frz_device* dev, const uint32_t* candidates_dev, const frz_sampl
   }
   DevStep s = host_step(position, tokens);
   fill_sampling(s, sampling);
-  if (int rc = device_put_step(dev, s)) return rc;
-  return device_finish(
-      dev, launch_draw(dev->stream, dev->step, candidates_dev, record_dev, nullptr),
-      "frz_op_draw");
+  return run_op(dev, s, "frz_op_draw", [&] {
+    return launch_draw(dev->stream, dev->step, candidates_dev, record_dev, nullptr);
+  });
 }
 
 int frz_op_numerics(frz_device* dev, int which, const float* in_dev, float* out_dev, int n) {
@@ -718,6 +734,8 @@ int frz_bench_gemv(frz_device* dev, const void* const* codes, const void* const*
   if (!shape_ok(rows, cols) || copies <= 0 || iters <= 0 || !us_per_launch) {
     return fail(FRZ_ERR_ARGUMENT, "frz_bench_gemv: bad argument");
   }
+  // The timed launches all read the device's step record.
+  std::lock_guard<std::mutex> lock(dev->ops);
   if (int rc = device_put_step(dev, host_step(0, 1))) return rc;
   return bench_graph(dev, copies, iters, graph, [&](int c) {
     return launch_gemv(dev->stream, dev->step, q4(codes[c], scales[c], rows, cols), x, cols, y,
@@ -732,6 +750,8 @@ int frz_bench_gated(frz_device* dev, const void* const* gate_codes,
   if (!shape_ok(rows, cols) || copies <= 0 || iters <= 0 || !us_per_launch) {
     return fail(FRZ_ERR_ARGUMENT, "frz_bench_gated: bad argument");
   }
+  // The timed launches all read the device's step record.
+  std::lock_guard<std::mutex> lock(dev->ops);
   if (int rc = device_put_step(dev, host_step(0, 1))) return rc;
   return bench_graph(dev, copies, iters, graph, [&](int c) {
     return launch_gated(dev->stream, dev->step, q4(gate_codes[c], gate_scales[c], rows, cols),

@@ -89,7 +89,9 @@ int frz_block_split(int format, const void* gguf_blocks, uint64_t blocks,
  *      tests do, tests/support/scratch_program.h:62-80) -----------------------
  * A Q4_0 matrix is `rows` rows of `cols` weights in the split layout above:
  * codes (rows * cols / 32 * 16 bytes) and scales (rows * cols / 32 halves).
- * `tokens` rows of input are processed from `position`. */
+ * `tokens` rows of input are processed from `position`. Ops through one
+ * handle may be called from several threads, while no model of that handle
+ * is at work: each runs whole, one after another on the device's stream. */
 
 /* y[t][o] = sum_k W[o][k] x[t][k] in the reference's order of addition
  * (src/core/kernels/matmul/matmul.wgsl:154-244, 390-465): the decode form
@@ -165,7 +167,8 @@ int frz_op_rope_attention(frz_device* dev, const float* qkv, const float* turns,
  * device holds until the process ends, so window and slots may reach at
  * most 224 chunks (14,272 keys; FRZ_ERR_ARGUMENT beyond). Every call on one
  * device shares that workspace, which keeps the last call's contents (each
- * call writes every state it reads): calls that overlap on one device race. */
+ * call writes every state it reads): calls that overlap through two handles
+ * to one device race. */
 int frz_op_rope_attention_noalloc(frz_device* dev, const float* qkv, const float* turns,
                                   const float* query_gain, const float* key_gain,
                                   uint16_t* key_cache, uint16_t* value_cache, float* out,
