@@ -358,7 +358,7 @@ hipError_t enqueue_readouts(frz_model* m) {
   for (int l = 0; l < count && e == hipSuccess; l += kReadoutRows) {
     const int rows = std::min(kReadoutRows, count - l);
     const DevStep* step = m->ro_steps + (rows == kReadoutRows ? 0 : 1);
-    mark(m, "readout", l);
+    mark(m, "readout", l + rows - 1);  // the batch's last layer
     NormArgs n{m->output_norm, nullptr, nullptr, m->store, m->ro_normed, c.epsilon, c.hidden, false};
     n.hidden_words = m->ro_words + l;
     e = launch_norm(s, step, n, rows);

@@ -914,8 +914,9 @@ int frz_program_mark_lost(frz_program* program);
  * "output.draw", and the capture store's "attention.capture",
  * "attention.weights", "ffn.capture", "readout", "output.readout". A launch of this backend
  * that runs several of the graph's roles (a product with its norm in its
- * prologue) names them all, joined by "+". A step's results are those of an
- * unprofiled one. */
+ * prologue) names them all, joined by "+". The readouts run in batches of up
+ * to 16 layers, each timed as one "readout" of the batch's last layer. A
+ * step's results are those of an unprofiled one. */
 typedef struct frz_launch_time {
   char role[96];
   uint32_t layer;        /* FRZ_NO_LAYER for the embedding and the output */

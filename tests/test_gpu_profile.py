@@ -12,8 +12,10 @@ import numpy as np
 import pytest
 
 import frizzle_amd as fz
+from frizzle_amd import graph
 from frizzle_amd import program as fprog
 from helpers import assert_same_bits
+from test_gpu_model import build_pair, small_config
 from test_gpu_program import _model, setup  # noqa: F401  (the fixture)
 
 pytestmark = pytest.mark.gpu
@@ -75,10 +77,24 @@ def test_profiled_prefill_step(device, setup, mode):
     b.close()
 
 
+def test_profiled_readouts_name_their_batch(device):
+    # 19 layers under the last one: a batch of 16, then one of 3, each timed
+    # as one launch of its last layer.
+    cfg = small_config(layers=20, vocab=1100)
+    model, _ = build_pair(device, cfg, seed=311)
+    model.set_capture(True)
+    prompt = np.random.default_rng(312).integers(0, cfg.vocab, 9).astype(np.uint32)
+    launches = model.profile_step(0, prompt, logits=True)
+    assert [layer for roles, layer, _ in launches if roles == "readout"] == [15, 18]
+    assert all(us > 0.0 for roles, _, us in launches)
+    model.close()
+
+
 def test_program_run_profiled(device, setup):
     cfg, path, plan = setup
     a, b = _model(device, plan, path), _model(device, plan, path)
     pa, pb = fprog.Program(a, plan), fprog.Program(b, plan)
+    order, _ = graph.gemma3_launches(plan)
     assert pa.can_profile and pa.launch_count > 0
     prompt = np.random.default_rng(303).integers(0, cfg.vocab, 300).astype(np.uint32)
     recs = [fprog.step_record(0, prompt, logits=True)]
@@ -102,6 +118,17 @@ def test_program_run_profiled(device, setup):
         # model reads.
         kept = [t["graph_index"] for t in launches if "readout" not in t["roles"]]
         assert kept == sorted(kept), kept
+        # Every launch, the readouts' batches among them: the graph's last
+        # launch of its roles in its layer.
+        for t in launches:
+            layer = graph.NO_LAYER if t["layer"] is None else t["layer"]
+            last = max(i for i, g in enumerate(order)
+                       if g.role in t["roles"].split("+") and g.layer == layer)
+            assert t["graph_index"] == last, t
+    # One batch of readouts, the prompt's end: layers 0 and 1, then the last
+    # layer's, the step's own candidates.
+    readouts = [(t["roles"], t["layer"]) for t in pa.profiles[0][3] if "readout" in t["roles"]]
+    assert readouts == [("output.readout", None), ("readout", cfg.layers - 2)], readouts
     # the prompt's step captures (the program turns the store on): its
     # capture launches are named too
     roles = {r for t in pa.profiles[0][3] for r in t["roles"].split("+")}
