@@ -168,3 +168,52 @@ def test_variants_start_from_the_prefix_rows_alone(device):
         for v, edits in enumerate(variants):
             assert np.array_equal(got[v], model.generate(prompt, edits, max_tokens=6)), (n, v)
     model.close()
+
+
+# Past 16 variants a step's products take several 16-token tiles, each row under
+# its own table: two tiles, one row into the second and third, and the most.
+@pytest.mark.parametrize("count,mixed", [(17, False), (33, True), (64, False)])
+def test_many_variants_are_the_replies_alone(device, count, mixed):
+    cfg = small_config()
+    if mixed:
+        model = fz.Model(device, cfg)
+        _set_all(model, _mixed_tensors(cfg, 71), MIXED)
+    else:
+        model, _ = build_pair(device, cfg, seed=71)
+    rng = np.random.default_rng(72 + count)
+    prompt = rng.integers(0, cfg.vocab, 40).astype(np.uint32)
+    variants = seeded_variants(cfg, rng, count)
+    samp = fz.sampling(temperature=1.0, top_k=64, top_p=1.0, min_p=0.0, seed=0x71)
+    got, res = model.generate_variants(prompt, variants, samp=samp, max_tokens=5, residuals=True)
+    for v, edits in enumerate(variants):
+        alone = model.generate(prompt, edits, samp=samp, max_tokens=5)
+        assert np.array_equal(got[v], alone), (v, got[v], alone)
+    # The last variant's residuals, a batch of its own: no row takes another's
+    # pins.
+    one, alone = model.generate_variants(prompt, variants[-1:], samp=samp, max_tokens=5,
+                                         residuals=True)
+    assert np.array_equal(one[0], got[-1])
+    n = len(one[0])
+    assert_same_bits(res[:n, :, -1], alone[:n, :, 0], "the last variant's residuals")
+    model.close()
+
+
+def test_variants_of_a_narrow_model(device):
+    # K of fewer groups than ranges (992): the gated product's wide tiles, a
+    # table a row.
+    cfg = small_config(hidden=992)
+    model, _ = build_pair(device, cfg, seed=81)
+    rng = np.random.default_rng(82)
+    prompt = rng.integers(0, cfg.vocab, 30).astype(np.uint32)
+    variants = seeded_variants(cfg, rng, 20)
+    got, res = model.generate_variants(prompt, variants, max_tokens=4, residuals=True)
+    for v, edits in enumerate(variants):
+        alone = model.generate(prompt, edits, max_tokens=4)
+        assert np.array_equal(got[v], alone), (v, got[v], alone)
+    for v in (7, 19):
+        _, alone = model.generate_variants(prompt, [variants[v]], max_tokens=4, residuals=True)
+        n = min(len(got[v]), res.shape[0])
+        assert_same_bits(res[:n, :, v], alone[:n, :, 0], f"variant {v}'s residuals")
+    # The pins act on their own rows alone.
+    assert sum(not np.array_equal(res[0, -1, 0], res[0, -1, v]) for v in range(1, 20)) >= 10
+    model.close()
