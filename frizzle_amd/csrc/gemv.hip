@@ -564,11 +564,12 @@ bool build_schedule(int groups, Schedule<NB>& S) {
 }
 
 // ---- a pass a wave ----------------------------------------------------------
-// A step of several rows (a batch of variants, a chat message, a prompt) makes one 16 x 16 tile per 16 output rows and 16 tokens. With a wave
-// a tile (gemm_ranges) its 32 ranges are one serial chain, which is all the
-// time there is until the tiles fill the chip: 55 us for gate and up and 51
-// for down at any 17 to 128 tokens. Here a workgroup takes a tile and its eight
-// waves a pass each. A pass is any four of the 32 ranges, chained in the four
+// A step of several rows (a batch of variants, a chat message, a prompt) makes
+// one 16 x 16 tile per 16 output rows and 16 tokens. With a wave a tile
+// (gemm_ranges) its 32 ranges are one serial chain, which is all the time there
+// is until the tiles fill the chip: 55 us for gate and up and 51 for down at
+// any 17 to 128 tokens. Here a workgroup takes a tile and its eight waves a
+// pass each; where that is the sooner is product_rules.h's to say. A pass is any four of the 32 ranges, chained in the four
 // blocks of one v_mfma_f32_16x16x1_4b_f32 per k; the range sums meet in LDS
 // by range index and are added in range order, so which ranges share a pass
 // changes no bit, and the host puts ranges of one length together: a pass
@@ -701,10 +702,11 @@ __device__ __forceinline__ void lds_reads_done() { __builtin_amdgcn_s_waitcnt(0x
 // one matrix (a pair of tiles on the same inputs).
 constexpr int kPlainKind = 0, kGatedKind = 1, kPairKind = 2;
 
-// Grid: x = 16-row tiles (32-row pairs); z = 16-token tiles (a row tile's
-// token tiles lie a multiple of eight workgroups apart for the model's
-// shapes, so on one XCD, whose L2 keeps the weights they share); y = the
-// halves of a split tile
+// Grid: x = 16-row tiles (32-row pairs); z = 16-token tiles (workgroups go to
+// the eight XCDs in turn, so a row tile's token tiles are on one XCD, whose L2
+// keeps the weights they share, where the x count is a multiple of eight, as
+// for Q/K/V, down and gate and up, and O in single tiles; O's 36 pairs have
+// every second token tile on another); y = the halves of a split tile
 // (HALVES = 2: the workgroup of half h takes passes 4 h .. 4 h + 3, which
 // hold ranges 16 h .. 16 h + 15; half 0 writes their prefix to y, half 1
 // each range's sum to parts). Rows past the end are read clamped and not
@@ -725,8 +727,10 @@ __global__ __launch_bounds__(kPassWaves / HALVES * 64, 4 / HALVES) void pass_til
   static_assert(!TWO || HALVES == 1, "two chains a lane combine in their workgroup");
   // Input slots, a wave's 8 KB each: one when a pass is at most two steps
   // (the second reuses it), else a ring of three for four waves or two for
-  // eight (the CU's 160 KB). Separate arrays, so that a read of one waits
-  // only for its own loads.
+  // eight (the CU's 160 KB). Two slots leave a CU one workgroup, so a long
+  // product's time steps up where its tiles pass the 256 CUs: down, 72 row
+  // tiles, takes 14.9 us at 48 tokens (216 workgroups) and 25.3 at 64 (288).
+  // Separate arrays, so that a read of one waits only for its own loads.
   constexpr int kSlots = STEPS >= 1 && STEPS <= 2 ? 1 : kWaves == 4 && STEPS > 0 ? 3 : 2;
   __shared__ __align__(16) float4 slot0[kWaves * kSlotFloat4s];
   __shared__ __align__(16) float4 slot1[kSlots > 1 ? kWaves * kSlotFloat4s : 1];
@@ -963,9 +967,10 @@ __global__ __launch_bounds__(kPassWaves / HALVES * 64, 4 / HALVES) void pass_til
 // LDS slot; both are double-buffered, step s + 1's fetched and decoded under
 // step s's products, with one barrier a step. A range opens on a product
 // with a zero addend, which is the chain's first fma.
-// 6,912 neurons over K = 1,152 took 215 us at 512 rows and 160 at 384 with a
-// wave a tile of two ranges; now 190 and 143 (86 TFLOP/s; the matrix cores
-// alone need 104 at 2.2 GHz, and 3.4 tiles a SIMD round up to 3.5).
+// 6,912 neurons over K = 1,152 took 219 us at 512 rows and 168 at 384 with a
+// wave a tile of two ranges; now 193 and 149 (84 TFLOP/s; the matrix cores
+// alone need 113 at the 2.2 GHz they hold, and 3.4 tiles a SIMD round up to
+// 3.5). Where it is taken is product_rules.h's to say.
 constexpr int kWideTokens = 32;  // a wave's tokens
 constexpr int kWideWaves = 4;
 constexpr int kWideGroups = 512;  // most groups of K

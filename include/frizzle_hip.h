@@ -95,7 +95,10 @@ int frz_block_split(int format, const void* gguf_blocks, uint64_t blocks,
 
 /* y[t][o] = sum_k W[o][k] x[t][k] in the reference's order of addition
  * (src/core/kernels/matmul/matmul.wgsl:154-244, 390-465): the decode form
- * when tokens == 1 or last_token, the tiled form otherwise. */
+ * when tokens == 1 or last_token, the tiled forms otherwise. Past 16 tokens
+ * cols may be at most 16,384 (32,768 while rows * tokens is under 786,432):
+ * FRZ_ERR_DEVICE beyond, before any product is launched; frz_op_gated, too,
+ * takes at most 16,384 past 16 tokens. */
 int frz_op_gemv(frz_device* dev, const void* codes, const void* scales,
                 int rows, int cols, const float* x, int x_stride, float* y,
                 int y_stride, uint32_t tokens, int last_token);
@@ -460,8 +463,11 @@ uint32_t frz_model_reused(const frz_model* model);
  * ends a prompt (a step asking for logits that is not a fed decode step)
  * writes every word of the store at its last row: Engine::inspect's and a
  * run's captures (src/core/capture/capture.h:15-34, :77-101), the store
- * laid out as frz_capture_layer says. It costs that step a head product,
- * a norm and a selection a layer for the readouts. */
+ * laid out as frz_capture_layer says. It costs that step a norm, a head
+ * product and a selection of 16 rows for every 16 layers' readouts, and the
+ * model, from the first time it is on until it is freed, those rows' logits
+ * and selection scratch beside the store (19 MB for Gemma-3-1B; a plan's
+ * buffers do not count them). */
 int frz_model_set_capture(frz_model* model, int enabled);
 /* The store's first `words` words, after the stream's work. */
 int frz_model_read_capture(frz_model* model, uint32_t* out, uint64_t words);

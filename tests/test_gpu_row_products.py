@@ -76,3 +76,40 @@ def test_gated_rows_bit_exact(device, rows, tokens, cols):
         return row
 
     _check_rows(da.numpy(), want, tokens)
+
+
+# Past 16 tokens a product's steps are held in a table: K past what it holds
+# is refused, before anything is launched, at every row count.
+@pytest.mark.parametrize("rows,cols,tokens,ok", [
+    (1536, 16384, 512, True), (1536, 16416, 512, False), (32, 32768, 17, True),
+    (32, 32800, 17, False), (32, 32800, 16, True)])
+def test_row_products_of_long_k(device, rows, cols, tokens, ok):
+    rng = np.random.default_rng(cols)
+    w = q4_blocks(rng, rows, cols)
+    codes, scales = _dev(device, 2, w)
+    x = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    dx, dy = device.array(x), device.array(np.full((tokens, rows), 7.0, np.float32))
+
+    def call():
+        fz._lib.check(fz.load().frz_op_gemv(device.handle, codes.ptr, scales.ptr, rows, cols,
+                                            dx.ptr, cols, dy.ptr, rows, tokens, 0))
+    if ok:
+        call()
+        for t in (0, tokens - 1):
+            assert_same_bits(dy.numpy()[t], orc.gemv_format(2, w, rows, cols, x[t]), f"token {t}")
+    else:
+        with pytest.raises(fz.FrzError):
+            call()
+        assert (dy.numpy() == 7.0).all()
+
+
+def test_gated_rows_of_long_k(device):
+    rows, cols = 32, 16416
+    rng = np.random.default_rng(2)
+    (gc, gs), (uc, us) = (_dev(device, 2, q4_blocks(rng, rows, cols)) for _ in range(2))
+    dx = device.array(rng.normal(0, 1, (17, cols)).astype(np.float32))
+    da = device.array(np.full((17, rows), 7.0, np.float32))
+    for tokens, ok in ((16, True), (17, False)):
+        rc = fz.load().frz_op_gated(device.handle, gc.ptr, gs.ptr, uc.ptr, us.ptr, rows, cols,
+                                    dx.ptr, da.ptr, tokens, 0, None, 0)
+        assert (rc == 0) == ok, tokens
