@@ -337,7 +337,7 @@ class Model:
         return toks, failed
 
     # A step's launches fit in this many entries (a prompt's last step with
-    # the capture store's readouts makes about 420 for Gemma-3-1B).
+    # the capture store's readouts makes about 300 for Gemma-3-1B).
     PROFILE_CAP = 2048
 
     def profile_step(self, position, ids, logits=False, samp=None):
