@@ -569,16 +569,17 @@ bool build_schedule(int groups, Schedule<NB>& S) {
 // (gemm_ranges) its 32 ranges are one serial chain, which is all the time there
 // is until the tiles fill the chip: 55 us for gate and up and 51 for down at
 // any 17 to 128 tokens. Here a workgroup takes a tile and its eight waves a
-// pass each; where that is the sooner is product_rules.h's to say. A pass is any four of the 32 ranges, chained in the four
-// blocks of one v_mfma_f32_16x16x1_4b_f32 per k; the range sums meet in LDS
-// by range index and are added in range order, so which ranges share a pass
-// changes no bit, and the host puts ranges of one length together: a pass
-// runs past a range's end only where the lengths mix. Each lane loads its
-// own operands straight from memory - its row's block of its range's group
-// and its token's 32 inputs of that group, which the matrix instruction reads
-// from the lane that loaded them - and a wave keeps its loads DEPTH steps
-// ahead of its products. Loads past a range's end read zeros through the
-// buffer resources' bounds: a zero input times a zero weight adds a zero.
+// pass each; where that is the sooner is product_rules.h's to say. A pass is
+// any four of the 32 ranges, chained in the four blocks of one
+// v_mfma_f32_16x16x1_4b_f32 per k; the range sums meet in LDS by range index
+// and are added in range order, so which ranges share a pass changes no bit,
+// and the host puts ranges of one length together: a pass runs past a range's
+// end only where the lengths mix. Each lane loads its own operands straight
+// from memory - its row's block of its range's group and its token's 32 inputs
+// of that group, which the matrix instruction reads from the lane that loaded
+// them - and a wave keeps its loads DEPTH steps ahead of its products. Loads
+// past a range's end read zeros through the buffer resources' bounds: a zero
+// input times a zero weight adds a zero.
 constexpr int kPassWaves = kRanges / 4;
 constexpr uint32_t kPastEnd = 0x40000000u;  // an offset past every buffer here
 
